@@ -120,8 +120,9 @@ int yhip_kv_fill_normal(yhip_ctx* ctx, int n_positions, unsigned long long seed)
  * tokens on), "attn_mfma" (1 = decode
  * attention on the matrix cores where head_dim % 32 == 0 and max_seq_len % 32 == 0, default;
  * 0 = the SIMT kernel), "bpc_qkv" / "bpc_o" / "bpc_w13" / "bpc_w2" / "bpc_lm" (workgroups per CU
- * of the decode matvecs, 0..16; 0 = the default: 2 for QKV, O and the lm_head, 12 for W1/W3, 1 for
- * W2; the results do not depend on it), "stats" (1 = time every synchronised step on the device
+ * of the decode matvecs, 0..16; 0 = the default: at dim 4096 2 for QKV, O and the lm_head and 12 for
+ * W1/W3, 1 for other rows of 2048 columns and more, 4 for shorter ones; the results do not depend
+ * on it), "stats" (1 = time every synchronised step on the device
  * with HIP events and reset the totals; 0 = off), "attn_o" (1 = default: for steps with at most
  * "attn_o_max" cached tokens (default 512), below max_seq_len, on the matrix-core attention's
  * shapes with at most 8 kv heads, attention and the O projection run in one launch whose

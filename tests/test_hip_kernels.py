@@ -98,6 +98,31 @@ def test_matvec_one_hot_is_exact(n):
         assert np.array_equal(hip().matvec(x, w), h2f(w[:, j]))
 
 
+@pytest.mark.parametrize("n", [8, 504, 512, 520, 1024, 1032, 2048, 2056, 4088, 4104, 8192, 8200, 12296, 16240])
+@pytest.mark.parametrize("d", [3, 2050])
+def test_matvec_row_lengths_at_the_piece_edges(n, d):
+    # Rows of any length go through the piece kernel (4096 and 14336 have their own): lengths around
+    # its staging sizes (1024, 2048, ... floats) and its pieces (1024, 2048 and 4096 columns), single
+    # rows (odd d) and pairs, more rows than one pass of the grid, against float64: a sum of n fp32
+    # products of random sign is off by about sqrt(n) 2^-24 of its largest partial sum, far inside
+    # RTOL. A one-hot input at the last column is exact, and an
+    # infinite one there stays an infinity (a chunk past the row adds 0 * 0, never 0 * inf).
+    rng = np.random.default_rng(n + d)
+    w = f16(rng.standard_normal((d, n)) * 0.05)
+    x = rng.standard_normal(n).astype(np.float32)
+    g = (1 + 0.1 * rng.standard_normal(n)).astype(np.float32)
+    r = rng.standard_normal(d).astype(np.float32)
+    w64 = h2f(w).astype(np.float64)
+    assert npref.rel_l2(hip().matvec(x, w, gain=g), w64 @ npref.rmsnorm(x, g, 1e-5)) < RTOL
+    assert npref.rel_l2(hip().matvec(x, w, resid=r), w64 @ x + r) < RTOL
+    x[:] = 0
+    x[-1] = 1
+    assert np.array_equal(hip().matvec(x, w), h2f(w[:, -1]))
+    w[:, -1] = f16(np.where(np.arange(d) % 2, 1.0, -1.0))
+    x[-1] = np.inf
+    assert np.array_equal(hip().matvec(x, w), np.where(np.arange(d) % 2, np.inf, -np.inf))
+
+
 @pytest.mark.parametrize("dim,hidden", [(64, 128), (256, 768), (4096, 14336)])
 @pytest.mark.parametrize("act", [1, 0])
 def test_ffn_parity(dim, hidden, act, bpc):

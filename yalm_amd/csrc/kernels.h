@@ -241,19 +241,10 @@ struct MatvecArgs {
   int track_max;
 };
 
-// Loads of one row segment for this lane: chunk c = lane + 64*u, u < KC (KC = K/512 when > 0).
-template <int KC, int R>
-__device__ __forceinline__ void load_group(u32x4 (&wv)[R][KC > 0 ? KC : 1], const uint16_t* const (&rows)[R], int lane) {
-#pragma unroll
-  for (int r = 0; r < R; ++r)
-#pragma unroll
-    for (int u = 0; u < KC; ++u)
-      wv[r][u] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(rows[r]) + lane + kWave * u);
-}
-
-// The same loads when the row pointers are wave-uniform (scalar registers): one buffer descriptor
-// per row in scalar registers and one shared lane offset, so no per-lane 64-bit addresses are
-// formed. Only for call sites whose group index is uniform by construction (readfirstlane).
+// Loads of one row segment per row of a group: lane l takes chunk l + 64*u, u < KC. The row pointers
+// are wave-uniform (scalar registers; the group index is uniform by construction, readfirstlane): one
+// buffer descriptor per row in scalar registers and one shared lane offset, so no per-lane 64-bit
+// addresses are formed.
 constexpr int kCpolNt = 2;  // cache-policy operand: nt (streaming)
 // valid == false: the descriptors cover no bytes and every load returns zero without a memory
 // access (the loads are still issued, so the caller's wait counts do not depend on a branch).
@@ -351,51 +342,10 @@ __device__ __forceinline__ void epilogue(const MatvecArgs& a, int p, const float
   }
 }
 
-// Stage the (optionally RMS-normalised) input vector into LDS: xs[i] = x[i] * inv * g[i] with
-// inv = 1/sqrt(mean(x^2) + eps) (reference src/infer.cpp:136-146), for any K % 4 == 0 (the
-// unrolled kernels stage through stage_load / stage_store below). x16: the fp16 embedding row as
-// the input instead of x. The step's RoPE table (head_dim floats) goes to LDS right after the vector.
-__device__ __forceinline__ void stage_input(const MatvecArgs& a, float* xs, float* red, const uint16_t* x16) {
-  if (a.rope_cs)
-    for (int i = threadIdx.x; i < a.head_dim; i += kBlock) xs[a.K + i] = a.rope_cs[i];
-  f32x4* o4 = reinterpret_cast<f32x4*>(xs);
-  const int n4 = a.K >> 2;
-  auto src4 = [&](int i) {
-    f32x4 v;
-    if (!x16) {
-      v = reinterpret_cast<const f32x4*>(a.x)[i];
-    } else {
-#pragma unroll
-      for (int e = 0; e < 4; ++e) v[e] = (float)__builtin_bit_cast(f16, x16[4 * i + e]);
-    }
-    return v;
-  };
-  if (a.gain) {
-    const f32x4* g4 = reinterpret_cast<const f32x4*>(a.gain);
-    float ss = 0.f;
-    for (int i = threadIdx.x; i < n4; i += kBlock) {
-      f32x4 v = src4(i);
-      ss += v[0] * v[0] + v[1] * v[1] + v[2] * v[2] + v[3] * v[3];
-    }
-    ss = block_sum(ss, red);
-    const float inv = 1.0f / sqrtf(ss / (float)a.K + a.eps);
-    for (int i = threadIdx.x; i < n4; i += kBlock) {
-      f32x4 v = src4(i), g = g4[i];
-      f32x4 o;
-      o[0] = v[0] * inv * g[0];
-      o[1] = v[1] * inv * g[1];
-      o[2] = v[2] * inv * g[2];
-      o[3] = v[3] * inv * g[3];
-      o4[i] = o;
-    }
-  } else {
-    for (int i = threadIdx.x; i < n4; i += kBlock) o4[i] = src4(i);
-  }
-  __syncthreads();
-}
-
-// The same staging in two halves, for the pipelined matvec (K == 1024*NPT, plain accesses):
-// stage_load issues every global read the staging needs (x or the raw fp16 embedding row, the
+// Staging of the (optionally RMS-normalised) input vector into LDS, xs[i] = x[i] * inv * g[i] with
+// inv = 1/sqrt(mean(x^2) + eps) (reference src/infer.cpp:136-146), in two halves (K == 1024*NPT;
+// any shorter K with the bounded form below); the step's RoPE table (head_dim floats) goes to LDS
+// right after the vector. stage_load issues every global read the staging needs (x or the raw fp16 embedding row, the
 // gains, the RoPE table) into registers; the caller then issues its first weight loads, and
 // stage_store normalises, fills LDS and synchronises the workgroup. Loads complete in issue order,
 // so consuming reads issued before the weights does not wait for the weights, and the first row
@@ -434,9 +384,11 @@ __device__ __forceinline__ void stage_load(const MatvecArgs& a, StagedInput<NPT,
   st.rc = a.rope_cs && (int)threadIdx.x < a.head_dim ? a.rope_cs[threadIdx.x] : 0.f;
 }
 
-template <int NPT, bool GAIN, bool EMB>
+// CUT: K may be shorter than 1024*NPT (stage_load_any read zeros past it).
+template <bool CUT = false, int NPT, bool GAIN, bool EMB>
 __device__ __forceinline__ void stage_store(const MatvecArgs& a, StagedInput<NPT, GAIN, EMB>& st, float* xs, float* red,
-                                            int pos, const uint16_t* x16) {
+                                            const uint16_t* x16) {
+  const int n4 = a.K >> 2;
   if (a.rope_cs && (int)threadIdx.x < a.head_dim) xs[a.K + threadIdx.x] = st.rc;
   if (EMB && x16) {
 #pragma unroll
@@ -460,11 +412,12 @@ __device__ __forceinline__ void stage_store(const MatvecArgs& a, StagedInput<NPT
       o[1] = st.xv[k][1] * inv * st.gv[k][1];
       o[2] = st.xv[k][2] * inv * st.gv[k][2];
       o[3] = st.xv[k][3] * inv * st.gv[k][3];
-      o4[threadIdx.x + kBlock * k] = o;
+      if (!CUT || (int)threadIdx.x + kBlock * k < n4) o4[threadIdx.x + kBlock * k] = o;
     }
   } else {
 #pragma unroll
-    for (int k = 0; k < NPT; ++k) o4[threadIdx.x + kBlock * k] = st.xv[k];
+    for (int k = 0; k < NPT; ++k)
+      if (!CUT || (int)threadIdx.x + kBlock * k < n4) o4[threadIdx.x + kBlock * k] = st.xv[k];
   }
   __syncthreads();
 }
@@ -485,8 +438,18 @@ __device__ __forceinline__ void track_rows(const MatvecArgs& a, int p, const flo
   }
 }
 
-// The fused matvec over groups p = blk*4 + wave + k*(nblk*4).
-// KC > 0: K == 512*KC*H, fully unrolled row streaming. KC == 0: any K % 8 == 0.
+// Embedding row as the input (reference src/infer.cpp:460-481: exact fp16 -> fp32), or null; workgroup
+// 0 also writes it out as fp32 where asked.
+__device__ __forceinline__ const uint16_t* embedding_input(const MatvecArgs& a, int blk) {
+  if (!a.emb) return nullptr;
+  const uint16_t* x16 = a.emb + (long)(a.token >= 0 ? a.token : a.params->token) * a.K;
+  if (a.emb_out && blk == 0)
+    for (int i = threadIdx.x; i < a.K; i += kBlock) a.emb_out[i] = (float)__builtin_bit_cast(f16, x16[i]);
+  return x16;
+}
+
+// The fused matvec over groups p = blk*4 + wave + k*(nblk*4), for K == 512*KC*H, fully unrolled row
+// streaming (other row lengths: matvec_any_body below).
 // H == 2 (R == 1 only): each row is streamed as two pieces of K/2 (see below).
 template <int KC, int R, EpiKind EPI, int H = 1>
 __device__ __forceinline__ RowMax matvec_body(const MatvecArgs& a, int blk, int nblk, float* lds) {
@@ -495,15 +458,8 @@ __device__ __forceinline__ RowMax matvec_body(const MatvecArgs& a, int blk, int 
   const int lane = threadIdx.x & (kWave - 1);
   const int wave = threadIdx.x / kWave;
   const int wave_stride = nblk * kWavesPerBlock;
-  int p = blk * kWavesPerBlock + wave;
   RowMax mx;
-  // embedding row as the input (reference src/infer.cpp:460-481: exact fp16 -> fp32)
-  const uint16_t* x16 = nullptr;
-  if (a.emb) {
-    x16 = a.emb + (long)(a.token >= 0 ? a.token : a.params->token) * a.K;
-    if (a.emb_out && blk == 0)
-      for (int i = threadIdx.x; i < a.K; i += kBlock) a.emb_out[i] = (float)__builtin_bit_cast(f16, x16[i]);
-  }
+  const uint16_t* x16 = embedding_input(a, blk);
 
   static_assert(H == 1 || (H == 2 && R == 1 && KC > 0), "two-piece rows: one row per group, unrolled");
   if constexpr (H == 2) {
@@ -531,7 +487,7 @@ __device__ __forceinline__ RowMax matvec_body(const MatvecArgs& a, int blk, int 
     __builtin_amdgcn_sched_barrier(0);
     issue(wa, 0, 0, n > 0);  // unconditional: a branch here would make the staging wait for it
     const int pos = EPI == kEpiQkvRope ? (a.pos >= 0 ? a.pos : a.params->pos) : 0;
-    stage_store(a, st, xs, red, pos, x16);
+    stage_store(a, st, xs, red, x16);
     float carry = 0.f;
     auto use = [&](const u32x4 (&wv)[1][KC], int i, int piece) {
       const float* xp = xs + piece * half;
@@ -565,7 +521,7 @@ __device__ __forceinline__ RowMax matvec_body(const MatvecArgs& a, int blk, int 
       use(wa, i, 0);
       use(wb, i, 1);
     }
-  } else if constexpr (KC > 0) {
+  } else {
     // Two register buffers, one group in flight: group i + 1's loads are issued as soon as group
     // i's have landed and before group i's dot products, reduction and epilogue, so a wave's
     // arithmetic overlaps its next memory round trip. (Two groups in flight per wave measured
@@ -589,7 +545,7 @@ __device__ __forceinline__ RowMax matvec_body(const MatvecArgs& a, int blk, int 
     __builtin_amdgcn_sched_barrier(0);
     issue(wa, prea, 0, n > 0);  // unconditional: a branch here would make the staging wait for it
     const int pos = EPI == kEpiQkvRope ? (a.pos >= 0 ? a.pos : a.params->pos) : 0;
-    stage_store(a, st, xs, red, pos, x16);
+    stage_store(a, st, xs, red, x16);
     auto use = [&](const u32x4 (&wv)[R][KC], const float (&pre)[R], int i) {
       const int pg = p0 + i * wave_stride;
       float acc[R];
@@ -623,30 +579,6 @@ __device__ __forceinline__ RowMax matvec_body(const MatvecArgs& a, int blk, int 
     } else if (i + 1 == n) {
       use(wa, prea, i);
     }
-  } else {
-    const int pos = EPI == kEpiQkvRope ? (a.pos >= 0 ? a.pos : a.params->pos) : 0;
-    stage_input(a, xs, red, x16);
-    const int nch = a.K >> 3;
-    for (; p < a.groups; p += wave_stride) {
-      const uint16_t* rows[R];
-      group_rows<R>(a, p, rows);
-      float pre[R];
-      epilogue_prefetch<R, EPI>(a, p, pre);
-      float acc[R];
-#pragma unroll
-      for (int r = 0; r < R; ++r) acc[r] = 0.f;
-      for (int c = lane; c < nch; c += kWave) {
-#pragma unroll
-        for (int r = 0; r < R; ++r) {
-          u32x4 w = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(rows[r]) + c);
-          acc[r] = dot8(w, xs + 8 * c, acc[r]);
-        }
-      }
-#pragma unroll
-      for (int r = 0; r < R; ++r) acc[r] = wave_sum(acc[r]);
-      epilogue<R, EPI>(a, p, acc, pre, pos, xs + a.K, lane == 0);
-      track_rows<R, EPI>(a, p, acc, mx);
-    }
   }
   return mx;
 }
@@ -655,6 +587,142 @@ template <int KC, int R, EpiKind EPI, int H = 1>
 __global__ void __launch_bounds__(kBlock) matvec_kernel(MatvecArgs a) {
   extern __shared__ float lds[];
   matvec_body<KC, R, EPI, H>(a, blockIdx.x, gridDim.x, lds);
+}
+
+// ------------------------------------------------------------------------------------------
+// The same matvec for any row length K <= 1024*NPT (K % 8 == 0): rows are streamed in pieces of KC
+// chunks per lane, the last piece cut by the buffer descriptor's size (a load past the row returns
+// zero without a memory access), so the pipeline of matvec_body (two register buffers, the next
+// piece issued before the current one is used, staging reads ahead of the first weights) holds for
+// every model width and not only for the unrolled 4096 and 14336. MULTI: rows of more than one piece.
+// A lane's chunk past the row multiplies its zero weights by the zero chunk at lds + 8, never by
+// whatever follows the input in LDS.
+// What it replaces (a rolled loop that waited for every 1 KB load before the next one, the input
+// staged before the first weights) was bound by that wait. Measured on MI355X, weights rotating
+// through 1 GiB, µs per launch before -> after (and TB/s): W2 4096 x 11008 48.2 -> 16.0 (5.6), W2
+// 2048 x 8192 18.8 -> 7.4 (4.5), W2 5120 x 13824 71.0 -> 23.8 (6.0), W1/W3 8192 x 2048 13.7 -> 12.2
+// (5.5), QKV 7168 x 5120 19.7 -> 14.6 (5.0), lm_head 32000 x 2048 27.8 -> 20.7 (6.3).
+// ------------------------------------------------------------------------------------------
+constexpr int any_chunks(int npt) { return npt >= 4 ? 8 : 2 * npt; }
+
+template <int NPT, bool GAIN, bool EMB>
+__device__ __forceinline__ void stage_load_any(const MatvecArgs& a, StagedInput<NPT, GAIN, EMB>& st, const uint16_t* x16) {
+  const int off = 16 * (int)threadIdx.x;
+  if (EMB && x16) {
+    const __amdgpu_buffer_rsrc_t rs =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(x16), 0, a.K * 2, kBufferConfig);
+#pragma unroll
+    for (int k = 0; k < NPT; ++k)
+      st.hv[k] = __builtin_bit_cast(unsigned long long,
+                                    __builtin_amdgcn_raw_buffer_load_b64(rs, off / 2 + 8 * kBlock * k, 0, 0));
+  } else {
+    const __amdgpu_buffer_rsrc_t rs =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(a.x), 0, a.K * 4, kBufferConfig);
+#pragma unroll
+    for (int k = 0; k < NPT; ++k)
+      st.xv[k] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, off + 16 * kBlock * k, 0, 0));
+  }
+  if (GAIN && a.gain) {
+    const __amdgpu_buffer_rsrc_t rs =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(a.gain), 0, a.K * 4, kBufferConfig);
+#pragma unroll
+    for (int k = 0; k < NPT; ++k)
+      st.gv[k] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, off + 16 * kBlock * k, 0, 0));
+  }
+  st.rc = a.rope_cs && (int)threadIdx.x < a.head_dim ? a.rope_cs[threadIdx.x] : 0.f;
+}
+
+template <int R, EpiKind EPI, int NPT>
+__device__ __forceinline__ RowMax matvec_any_body(const MatvecArgs& a, int blk, int nblk, float* lds) {
+  constexpr int KC = any_chunks(NPT);
+  constexpr bool MULTI = NPT > 4;  // K > 512 * KC
+  float* red = lds;                // kWavesPerBlock floats; floats 8..15 stay zero
+  float* xs = lds + 16;            // K floats (+ the RoPE table)
+  const int lane = threadIdx.x & (kWave - 1);
+  const int wave_stride = nblk * kWavesPerBlock;
+  RowMax mx;
+  const uint16_t* x16 = embedding_input(a, blk);
+  const int p0 = blk * kWavesPerBlock + __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int n = p0 < a.groups ? (a.groups - 1 - p0) / wave_stride + 1 : 0;  // this wave's groups
+  const int nch = a.K >> 3;
+  const int np = MULTI ? (nch + kWave * KC - 1) / (kWave * KC) : 1;  // pieces per row
+  const int items = n * np;
+  u32x4 wa[R][KC], wb[R][KC];
+  float prea[R], preb[R];
+  int ig = 0, ip = 0;  // group and piece of the next issue
+  auto issue = [&](u32x4 (&wv)[R][KC], float (&pre)[R], bool valid = true) {
+    const uint16_t* rows[R];
+    const int g = valid ? p0 + ig * wave_stride : 0;
+    group_rows<R>(a, g, rows);
+    const int done = ip * KC * 1024;  // bytes of the row before this piece
+    const int left = valid ? min(a.K * 2 - done, KC * 1024) : 0;
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+          const_cast<uint16_t*>(rows[r]) + done / 2, 0, left, kBufferConfig);
+#pragma unroll
+      for (int u = 0; u < KC; ++u)
+        wv[r][u] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, lane * 16, u * 1024, kCpolNt));
+    }
+    epilogue_prefetch<R, EPI>(a, g, pre);
+    if (!MULTI || ++ip == np) {
+      ip = 0;
+      ++ig;
+    }
+  };
+  StagedInput<NPT, kEpiGain<EPI>, kEpiEmb<EPI>> st;
+  stage_load_any(a, st, x16);
+  __builtin_amdgcn_sched_barrier(0);
+  issue(wa, prea, n > 0);  // unconditional: a branch here would make the staging wait for it
+  const int pos = EPI == kEpiQkvRope ? (a.pos >= 0 ? a.pos : a.params->pos) : 0;
+  if (threadIdx.x < 8) lds[8 + threadIdx.x] = 0.f;
+  stage_store<true>(a, st, xs, red, x16);
+  int ug = 0, up = 0;  // group and piece of the next use
+  float acc[R] = {};
+  auto use = [&](const u32x4 (&wv)[R][KC], const float (&pre)[R]) {
+    const int c0 = up * KC * kWave + lane;
+#pragma unroll
+    for (int u = 0; u < KC; ++u) {
+      const int c = c0 + kWave * u;
+      const float* xp = c < nch ? xs + 8 * c : lds + 8;
+#pragma unroll
+      for (int r = 0; r < R; ++r) acc[r] = dot8(wv[r][u], xp, acc[r]);
+      if ((u & 3) == 3) __builtin_amdgcn_sched_barrier(0);
+    }
+    if (MULTI && ++up < np) return;
+    up = 0;
+#pragma unroll
+    for (int r = 0; r < R; ++r) acc[r] = wave_sum(acc[r]);
+    const int pg = p0 + ug++ * wave_stride;
+    epilogue<R, EPI>(a, pg, acc, pre, pos, xs + a.K, lane == 0);
+    track_rows<R, EPI>(a, pg, acc, mx);
+#pragma unroll
+    for (int r = 0; r < R; ++r) acc[r] = 0.f;
+  };
+  int i = 0;
+  for (; i + 2 < items; i += 2) {
+    issue(wb, preb);
+    __builtin_amdgcn_sched_barrier(0);
+    use(wa, prea);
+    issue(wa, prea);
+    __builtin_amdgcn_sched_barrier(0);
+    use(wb, preb);
+  }
+  if (i + 2 == items) {
+    issue(wb, preb);
+    __builtin_amdgcn_sched_barrier(0);
+    use(wa, prea);
+    use(wb, preb);
+  } else if (i + 1 == items) {
+    use(wa, prea);
+  }
+  return mx;
+}
+
+template <int R, EpiKind EPI, int NPT>
+__global__ void __launch_bounds__(kBlock) matvec_any_kernel(MatvecArgs a) {
+  extern __shared__ float lds[];
+  matvec_any_body<R, EPI, NPT>(a, blockIdx.x, gridDim.x, lds);
 }
 
 // Packed (logit, index) whose unsigned order is the argmax order with the reference's tie rule
@@ -691,6 +759,12 @@ template <int KC>
 __global__ void __launch_bounds__(kBlock) lm_head_argmax_kernel(MatvecArgs a, unsigned long long* key) {
   extern __shared__ float lds[];
   const RowMax mx = matvec_body<KC, 2, kEpiStore>(a, blockIdx.x, gridDim.x, lds);
+  argmax_post(mx, key);
+}
+template <int NPT>
+__global__ void __launch_bounds__(kBlock) lm_head_argmax_any_kernel(MatvecArgs a, unsigned long long* key) {
+  extern __shared__ float lds[];
+  const RowMax mx = matvec_any_body<2, kEpiStore, NPT>(a, blockIdx.x, gridDim.x, lds);
   argmax_post(mx, key);
 }
 

@@ -215,14 +215,19 @@ std::vector<float> make_inv_freq(int head_dim, int rotary_dim, float theta) {
 // ---- matvec launch -------------------------------------------------------------------------
 // Workgroups per CU, measured best on MI355X in the decode step: 2 for 4096-long rows (QKV, O,
 // lm_head), 1 for 14336-long rows (W2, whose 57 KB LDS input already limits residency), and 12 for
-// W1/W3 + SwiGLU. With 149 VGPRs three of its workgroups fit a CU, so a 12-per-CU grid (about one
-// row pair per wave) leaves most workgroups queued, and the hardware dispatcher hands each CU a new
-// one as soon as one finishes: the CUs whose loads are served late simply take fewer. That
-// balances the launch's tail (2.621 -> 2.570 ms per token); 2-8 per CU are in between, 14 and 16
+// W1/W3 + SwiGLU on 4096-long rows. With 149 VGPRs three of its workgroups fit a CU, so a 12-per-CU
+// grid (about one row pair per wave) leaves most workgroups queued, and the hardware dispatcher hands
+// each CU a new one as soon as one finishes: the CUs whose loads are served late simply take fewer.
+// That balances the launch's tail (2.621 -> 2.570 ms per token); 2-8 per CU are in between, 14 and 16
 // no better.
+// Other row lengths (matvec_any_kernel): one workgroup per CU from 2048 columns on, so the input is
+// staged once per CU (µs with 1 / 2 / 12 per CU: QKV 7168 x 5120 14.6 / 15.6 / 16.1, W1/W3 13824 x 5120
+// 44.4 / 44.6 / 48.0, W1/W3 8192 x 2048 12.2 / 12.4 / 12.6, W2 2048 x 8192 7.4 / 7.9 / 7.9), four on
+// shorter rows, whose staging is nothing beside the waves' own latency (lm_head 32000 x 256 with
+// 1 / 2 / 4 / 12: 9.6 / 7.2 / 6.6 / 7.3).
 int default_bpc(int K, int kind = -1) {
-  if (kind == kEpiSwiGLU) return 12;
-  return K >= 8192 ? 1 : 2;
+  if (K == 4096) return kind == kEpiSwiGLU ? 12 : 2;
+  return K >= 2048 ? 1 : 4;
 }
 
 template <int KC, int R, EpiKind EPI, int H = 1>
@@ -232,15 +237,29 @@ void launch_mv(const MatvecArgs& a, int blocks, hipStream_t s) {
   hipLaunchKernelGGL((matvec_kernel<KC, R, EPI, H>), dim3(blocks), dim3(kBlock), lds, s, a);
 }
 
+// Row lengths other than the unrolled ones: the smallest staging (NPT float4 per thread) that holds K.
+template <int R, EpiKind EPI>
+void launch_mv_any(const MatvecArgs& a, int blocks, hipStream_t s) {
+  const size_t lds = (16 + (size_t)a.K + (a.rope_cs ? (size_t)a.head_dim : 0)) * sizeof(float);
+  auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3(blocks), dim3(kBlock), lds, s, a); };
+  if (a.K <= 1024) go(matvec_any_kernel<R, EPI, 1>);
+  else if (a.K <= 2048) go(matvec_any_kernel<R, EPI, 2>);
+  else if (a.K <= 4096) go(matvec_any_kernel<R, EPI, 4>);
+  else if (a.K <= 8192) go(matvec_any_kernel<R, EPI, 8>);
+  else go(matvec_any_kernel<R, EPI, 16>);
+}
+
 template <EpiKind EPI>
 void launch_by_shape(const MatvecArgs& a, int R, int blocks, hipStream_t s) {
-  if (R == 1) {
-    if (a.K == 4096) launch_mv<8, 1, EPI>(a, blocks, s);
-    else if (a.K == 14336) launch_mv<14, 1, EPI, 2>(a, blocks, s);  // two 7168-long pieces per row
-    else launch_mv<0, 1, EPI>(a, blocks, s);
+  if (R == 1) {  // launch_matvec refuses single rows for the epilogues that work on pairs
+    if constexpr (EPI == kEpiStore || EPI == kEpiResidual) {
+      if (a.K == 4096) launch_mv<8, 1, EPI>(a, blocks, s);
+      else if (a.K == 14336) launch_mv<14, 1, EPI, 2>(a, blocks, s);  // two 7168-long pieces per row
+      else launch_mv_any<1, EPI>(a, blocks, s);
+    }
   } else {
     if (a.K == 4096) launch_mv<8, 2, EPI>(a, blocks, s);
-    else launch_mv<0, 2, EPI>(a, blocks, s);
+    else launch_mv_any<2, EPI>(a, blocks, s);
   }
 }
 
@@ -268,6 +287,7 @@ int launch_matvec(yhip_ctx* ctx, MatvecArgs a, int kind, int R, int num_cus, hip
   if (a.K % 8 != 0 || (16 + (size_t)a.K + 128) * sizeof(float) > 65536)
     return fail(ctx, YHIP_EINVAL, "matvec: row length must be a multiple of 8 and at most 16240");
   if (R != 1 && R != 2) return fail(ctx, YHIP_EINVAL, "matvec: R must be 1 or 2");
+  if (R == 1 && kind != kEpiStore && kind != kEpiResidual) return fail(ctx, YHIP_EINVAL, "matvec: this epilogue takes row pairs");
   if (kind == kEpiResidual && (a.gain || a.emb)) return fail(ctx, YHIP_EINVAL, "matvec: the residual epilogue takes no gain or embedding input");
   if (kind == kEpiSwiGLU && a.emb) return fail(ctx, YHIP_EINVAL, "matvec: the SwiGLU epilogue takes no embedding input");
   if (kind == kEpiQkvRope && !a.rope_cs) return fail(ctx, YHIP_EINVAL, "matvec: the RoPE epilogue takes a precomputed table (rope_cs)");
@@ -574,10 +594,15 @@ int enqueue_step(yhip_ctx* ctx, int mode, int variant) {
     const int bpc = ctx->mv_bpc[4] > 0 ? ctx->mv_bpc[4] : default_bpc(a.K);
     const int blocks = std::max(1, std::min((a.groups + kWavesPerBlock - 1) / kWavesPerBlock, ctx->num_cus * bpc));
     const size_t lds = (16 + (size_t)a.K) * sizeof(float);
-    if (a.K == 4096)
-      hipLaunchKernelGGL(lm_head_argmax_kernel<8>, dim3(blocks), dim3(kBlock), lds, s, a, ctx->argmax_key);
-    else
-      hipLaunchKernelGGL(lm_head_argmax_kernel<0>, dim3(blocks), dim3(kBlock), lds, s, a, ctx->argmax_key);
+    auto go = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, dim3(blocks), dim3(kBlock), lds, s, a, ctx->argmax_key);
+    };
+    if (a.K == 4096) go(lm_head_argmax_kernel<8>);
+    else if (a.K <= 1024) go(lm_head_argmax_any_kernel<1>);
+    else if (a.K <= 2048) go(lm_head_argmax_any_kernel<2>);
+    else if (a.K <= 4096) go(lm_head_argmax_any_kernel<4>);
+    else if (a.K <= 8192) go(lm_head_argmax_any_kernel<8>);
+    else go(lm_head_argmax_any_kernel<16>);
     HIP_TRY(ctx, hipGetLastError());
   }
   if (mode == 1) {
