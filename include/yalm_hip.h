@@ -210,7 +210,7 @@ int yhip_test_gemm(const uint16_t* a, const uint16_t* b, const uint16_t* b3, int
                    float* c, uint16_t* h);
 /* The prefill GEMM variant yhip_prefill runs for this shape and mode (as yhip_test_gemm), under the
  * current process-wide options: stages 6 = the eight-wave 256 x 256 kernel, 2..4 = the LDS
- * pipeline's depth; bk the k-step; bm the workgroup's rows. No
+ * pipeline's depth, 1 = the weight-streaming kernel (up to 128 rows, K a multiple of 128); bk the k-step; bm the workgroup's rows. No
  * reference counterpart (the reference has no batched prefill). */
 int yhip_gemm_variant(int M, int N, int K, int mode, int* stages, int* bk, int* bm);
 /* Greedy argmax on the device with the reference tie rule. */

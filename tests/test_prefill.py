@@ -66,6 +66,30 @@ def test_gemm_swiglu(M, N, K, gemm_variant):
     assert npref.rel_l2(got, want) < 2e-3  # fp16 output
 
 
+@pytest.mark.parametrize("M", [1, 31, 33, 64, 65, 96, 97, 128])
+@pytest.mark.parametrize("N,K", [(8, 128), (101, 384), (264, 1664), (16600, 256)])
+def test_gemm_weight_streaming(M, N, K):
+    # Up to 128 rows with K % 128 == 0: row counts around the kernel's 32-row steps, N around its
+    # 16-row tiles and 128-row workgroups (101: rows of outputs that are no multiple of 4), spans of
+    # fewer stages than its ring (K 128, 256, 384), 13 stages over 13 splits (264 x 1664: one each;
+    # fp32 partials) and no split (16600 rows: more weight blocks than CUs). fp32 sums of up to 1664
+    # products: 1e-6 is 16 roundings of the result.
+    H = hip()
+    assert H.gemm_variant(M, N, K, 0) == (1, 128, (M + 31) // 32 * 32)
+    rng = np.random.default_rng(M + N + K)
+    a = f16(rng.standard_normal((M, K)))
+    b = f16(rng.standard_normal((N, K)) * 0.05)
+    b3 = f16(rng.standard_normal((N, K)) * 0.05)
+    A = h2f(a).astype(np.float64)
+    want = A @ h2f(b).astype(np.float64).T
+    u = A @ h2f(b3).astype(np.float64).T
+    c0 = rng.standard_normal((M, N)).astype(np.float32)
+    assert npref.rel_l2(H.gemm(a, b, mode=0), want) < 1e-6
+    assert npref.rel_l2(H.gemm(a, b, mode=1, c=c0), c0 + want) < 1e-6
+    got = h2f(H.gemm(a, b, mode=2, b3=b3))
+    assert npref.rel_l2(got, want / (1 + np.exp(-want)) * u) < 2e-3  # fp16 output
+
+
 @pytest.mark.parametrize("ksplit", [2, 4, 8])
 @pytest.mark.parametrize("M,N,K", [(37, 192, 1024), (128, 256, 4096), (200, 128, 512)])
 def test_gemm_split_k(M, N, K, ksplit):

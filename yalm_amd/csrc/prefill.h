@@ -330,6 +330,186 @@ __global__ void __launch_bounds__(256) gemm_splitk_reduce(GemmArgs g) {
   }
 }
 
+// ------------------------------------------------------------------------------------------
+// Weight-streaming GEMM for short prompts (up to kStreamRows rows): the launch is bound by reading B
+// once from HBM, so B goes straight from memory into registers and only the activations pass
+// through LDS. v_mfma_f32_16x16x32_f16 with the weights as the A operand: the accumulator holds four
+// consecutive outputs of one activation row (16-byte stores).
+// A wave owns a tile of 16 weight rows (SwiGLU: 8 rows of W1 and the same 8 of W3) times all BM
+// activation rows, a workgroup of eight waves 128 weight rows. A load instruction covers whole 128-byte
+// lines, 8 of them per row pair half: lane l reads chunk 2 (l / 16) + (l / 8) % 2 of row l % 8, and
+// the loads of a tile's rows 0-7 and 8-15 are exchanged between lanes l and l ^ 8 (one DPP move per
+// register) into the MFMA's operand, row l % 16 with one k chunk per 16 lanes. In the operand's own
+// order an instruction reads 64 bytes of each of 16 rows; memory-only, W1/W3 at the 7B shape then
+// takes 43-48 us against 37.9 us with whole lines (W2 21.4 against 19.3).
+// k advances in stages of 128: a ring of four stages, three of them in flight while one is used.
+// Each stage orders its activation copies (global_load_lds, [BM][128] halves with chunk c of row r
+// at position c ^ (r % 16): the 16 rows of a fragment read fall in distinct banks) before its weight
+// loads, so one vmcnt wait covers both and the barrier behind it publishes the activations. Stages
+// past the end re-read the last activations and load weights through an empty descriptor, so every
+// iteration has the same loads in flight.
+// K % 128 == 0. Against the LDS pipeline (which keeps one 16 KB weight stage per workgroup in flight),
+// us per launch in a 7B prefill: 32 rows W1/W3 68.0 -> 45.7 (5.1 TB/s), W2 32.1 -> 22.1, QKV 19.2 -> 12.6,
+// O 15.2 -> 10; 61 rows 69.2 -> 48.7, 34.0 -> 25.9, 20.6 -> 15.8. What is left above the pattern's
+// 37.9 us is one workgroup per CU meeting at a barrier per stage (at 128 rows also the activations'
+// fragment reads: 8 KB of LDS per 1 KB of weights).
+// ------------------------------------------------------------------------------------------
+__device__ __forceinline__ f32x4 mfma16(u32x4 a, u32x4 b, f32x4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8, a), __builtin_bit_cast(half8, b), c, 0, 0, 0);
+}
+// row[n .. n + 3] = or += v, columns past N left out; one 16-byte access where the row length allows.
+__device__ __forceinline__ void store4(float* row, int n, int N, long ld, f32x4 v, bool add) {
+  if (n + 3 < N && ld % 4 == 0 && N % 4 == 0) {
+    f32x4* p = reinterpret_cast<f32x4*>(row + n);
+    *p = add ? *p + v : v;
+  } else {
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if (n + e < N) row[n + e] = add ? row[n + e] + v[e] : v[e];
+  }
+}
+constexpr int kStreamK = 128;     // k per stage
+constexpr int kStreamRows = 128;  // most activation rows
+constexpr int kStreamWaves = 8;
+
+// Lanes 8-15 of every 16 take `src` of lane ^ 8, the others keep `keep` (HIGH), or the reverse.
+template <bool HIGH>
+__device__ __forceinline__ u32x4 swap8(u32x4 keep, u32x4 src) {
+  u32x4 r;
+#pragma unroll
+  for (int d = 0; d < 4; ++d)
+    r[d] = (uint32_t)__builtin_amdgcn_update_dpp((int)keep[d], (int)src[d], 0x128 /* row_ror:8 */, 0xf,
+                                                 HIGH ? 0xc : 0x3, false);
+  return r;
+}
+
+// Output columns per workgroup.
+constexpr int stream_cols(int epi) { return kStreamWaves * (epi == kGemmSwiGLU ? 8 : 16); }
+
+template <int EPI, int BM>
+__global__ void __launch_bounds__(64 * kStreamWaves) gemm_stream_kernel(GemmArgs g) {
+  constexpr int NW = kStreamWaves;
+  static_assert(BM % (4 * NW) == 0 && BM <= kStreamRows, "activation rows");
+  constexpr int S = 4;               // ring of stages
+  constexpr int MT = BM / 16;        // 16-row activation tiles
+  constexpr int NA = BM / (4 * NW);  // activation copies per wave and stage (4 rows of 256 bytes each)
+  constexpr int LPS = NA + 4;        // loads per wave and stage
+  constexpr int TC = EPI == kGemmSwiGLU ? 8 : 16;  // output columns per tile
+  constexpr int NC = stream_cols(EPI);
+  __shared__ __attribute__((aligned(1024))) uint16_t As[S][BM * kStreamK];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int ks = g.ksplit > 1 ? g.ksplit : 1;
+  int tm, tn, split;
+  if (!gemm_unit(1, (g.N + NC - 1) / NC, ks, tm, tn, split)) return;
+  const int T = g.K / kStreamK;
+  const int s0 = (int)((long)split * T / ks), s1 = (int)((long)(split + 1) * T / ks);
+
+  // activation copies: instruction j of this wave fills rows 4 (wave + NW j) .. + 3 of the stage
+  const uint16_t* arow[NA];
+#pragma unroll
+  for (int j = 0; j < NA; ++j) {
+    const int r = 4 * (wave + NW * j) + (lane >> 4);
+    arow[j] = g.A + (long)min(r, g.M - 1) * g.lda + 8 * ((lane & 15) ^ (r & 15));
+  }
+  // the wave's weight tile: first output column, and this lane's byte offsets of its two row halves
+  const int nb = tn * NC + wave * TC;
+  unsigned voff[2];
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const int row = nb + (EPI == kGemmSwiGLU ? 0 : 8 * h) + (lane & 7);
+    voff[h] = (unsigned)min(row, g.N - 1) * (unsigned)(g.ldb * 2) + 16u * (2 * (lane >> 4) + ((lane >> 3) & 1));
+  }
+  const unsigned bytes = (unsigned)g.N * (unsigned)(g.ldb * 2);
+  u32x4 w[S][2][2];  // [slot][128-byte line][row half]
+  auto issue = [&](int slot, int st) {
+    const int ka = min(st, s1 - 1) * kStreamK;
+#pragma unroll
+    for (int j = 0; j < NA; ++j) load_lds16(arow[j] + ka, &As[slot][(wave + NW * j) * 512]);
+    const int kw = st * kStreamK * 2, n = st < s1 ? (int)bytes : 0;
+    const __amdgpu_buffer_rsrc_t r0 =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(g.B), 0, n, kBufferConfig);
+    const __amdgpu_buffer_rsrc_t r1 = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<uint16_t*>(EPI == kGemmSwiGLU ? g.B3 : g.B), 0, n, kBufferConfig);
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+      w[slot][c][0] =
+          __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(r0, voff[0], kw + 128 * c, kCpolNt));
+      w[slot][c][1] =
+          __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(r1, voff[1], kw + 128 * c, kCpolNt));
+    }
+  };
+  f32x4 acc[MT];
+#pragma unroll
+  for (int i = 0; i < MT; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const int frow = (lane & 15) * kStreamK;
+  auto step = [&](int slot, int st) {
+    wait_vmcnt<2 * LPS>();  // stage st has landed (two later ones may be outstanding)
+    __builtin_amdgcn_sched_barrier(0);
+    __asm__ volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();  // for every wave; stage st - 1 is no longer read
+    __asm__ volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+    issue((slot + 3) % S, st + 3);
+    __builtin_amdgcn_sched_barrier(0);
+    if (st >= s1) return;
+#pragma unroll
+    for (int kk = 0; kk < 4; ++kk) {  // line kk / 2, even or odd chunks
+      u32x4 fa[MT];
+      const int pos = 8 * ((8 * (kk >> 1) + 2 * (lane >> 4) + (kk & 1)) ^ (lane & 15));
+#pragma unroll
+      for (int i = 0; i < MT; ++i) fa[i] = *reinterpret_cast<const u32x4*>(&As[slot][i * 16 * kStreamK + frow + pos]);
+      const u32x4 lo = w[slot][kk >> 1][0], hi = w[slot][kk >> 1][1];
+      const u32x4 fw = (kk & 1) ? swap8<false>(hi, lo) : swap8<true>(lo, hi);
+#pragma unroll
+      for (int i = 0; i < MT; ++i) acc[i] = mfma16(fw, fa[i], acc[i]);
+    }
+  };
+  issue(0, s0);
+  issue(1, s0 + 1);
+  issue(2, s0 + 2);
+  for (int st = s0; st < s1; st += 4) {
+    step(0, st);
+    step(1, st + 1);
+    step(2, st + 2);
+    step(3, st + 3);
+  }
+  wait_vmcnt<0>();  // the copies past the end have landed before the LDS is given back
+
+  // lane l: tile rows 4 (l / 16) .. + 3 of activation row 16 i + l % 16
+#pragma unroll
+  for (int i = 0; i < MT; ++i) {
+    const int m = i * 16 + (lane & 15);
+    if (m >= g.M) continue;
+    if constexpr (EPI == kGemmSwiGLU) {  // lanes 0-31 hold W1, the same outputs of W3 are 32 lanes on
+      const int n = nb + 4 * ((lane >> 4) & 1);
+      if (ks > 1) {
+        store4(g.P + ((long)split * g.M + m) * (2L * g.N) + (lane < 32 ? 0 : g.N), n, g.N, 2L * g.N, acc[i], false);
+        continue;
+      }
+      uint16_t h[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float a1 = acc[i][e], a3 = half_swap_other(a1);
+        h[e] = __builtin_bit_cast(uint16_t, (f16)((g.act == 1 ? silu_fast(a1) : gelu(a1)) * a3));
+      }
+      if (lane >= 32) continue;
+      uint16_t* hp = g.H + (long)m * g.ldh + n;
+      if (n + 3 < g.N && g.ldh % 4 == 0) {
+        *reinterpret_cast<unsigned long long*>(hp) = (unsigned long long)h[0] | (unsigned long long)h[1] << 16 |
+                                                     (unsigned long long)h[2] << 32 | (unsigned long long)h[3] << 48;
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (n + e < g.N) hp[e] = h[e];
+      }
+    } else {
+      const int n = nb + 4 * (lane >> 4);
+      if (ks > 1) store4(g.P + ((long)split * g.M + m) * g.N, n, g.N, g.N, acc[i], false);
+      else store4(g.C + (long)m * g.ldc, n, g.N, g.ldc, acc[i], EPI == kGemmResid);
+    }
+  }
+}
+
 constexpr int kBigM = 256, kBigN = 256;
 
 // Partial slots and flags of the eight-wave kernel's split round: a slot holds one 256 x 256 fp32

@@ -33,10 +33,6 @@ thread_local std::string g_thread_err;
 // yhip_set_option(NULL, "test_bpc", n) so tests can force many row groups per wave.
 int g_test_bpc = 0;
 bool g_attn_mfma = true;  // attention kernel of the kernel-level entry points (process-wide option)
-// Large-tile prefill GEMM k-step schedule (BigTile::mainloop<IL>): 0 = the compiler's own order,
-// 1 = copies and fragment reads placed between the MFMAs by scheduling groups, 2 = fenced phases;
-// -1 (default) = per shape: 2 for K >= 8192, else 1. Same box, 3200 rows (us): W1/W3 962 / 890 /
-// 905, W2 510 / 488 / 463.
 int g_gemm_ppsplit = 1;   // eight-wave prefill GEMM: split the last, partial round of tiles along K
 int g_gemm_stages = 4;    // prefill GEMM: LDS pipeline depth 2..4, or 6 = the eight-wave kernel
 int g_gemm_bk = 32;       // prefill GEMM: k-step of the LDS pipeline (32 or 64)
@@ -811,8 +807,6 @@ int run_step_inner(yhip_ctx* ctx, int token, int pos, int mode) {
 }
 
 // ---- batched prefill ---------------------------------------------------------------------------
-// The prefill GEMM variant for an epilogue and shape (stages 1 = the 256 x 256 kernel, 2..4 the
-// LDS pipeline's depth, 0 the register-staged kernel), or the forced process-wide one.
 // Split of the eight-wave GEMM's last, partial round (tiles % CUs of them; the kernel's PPSplit):
 // with more of those tiles than half the CUs, one tail piece per tile, the idle CUs taking q of
 // them each and the main parts' k-range kd balancing the two (W1/W3 at 3200 rows: 176 tiles after
@@ -853,11 +847,25 @@ PPSplit pp_split_plan(long tiles, int KI, int P, bool workspace) {
   return sp;
 }
 
+// Whether the weight-streaming kernel takes a shape: whole stages of k, all rows in one tile, weights
+// within a buffer descriptor's 32-bit offsets.
+bool stream_fits(int M, int N, int K) { return M <= kStreamRows && K % kStreamK == 0 && (long)N * K < (1L << 31); }
+
+// The prefill GEMM variant for an epilogue and shape (stages 1 = the weight-streaming kernel, 2..4 the
+// LDS pipeline's depth, 6 = the eight-wave 256 x 256 kernel), or the forced process-wide one.
 void gemm_choice(int epi, int M, int N, int K, int cus, int& stages, int& bk, int& bm) {
   stages = g_gemm_stages;
   bk = g_gemm_bk;
   bm = g_gemm_bm;
   if (!g_gemm_auto) return;
+  // Up to 128 rows the launch is bound by the weights: the streaming kernel (8 layers of the 7B shape,
+  // us per prefill of 16 / 32 / 64 / 96 / 128 tokens: 1440 / 1483 / 1583 / 1631 / 1666 with the LDS
+  // pipeline, 1069 / 1111 / 1268 / 1434 / 1582 with it).
+  // A forced K split is the LDS pipeline's.
+  if (stream_fits(M, N, K) && g_gemm_ksplit == 0) {
+    stages = 1;
+    return;
+  }
   // Variant per shape, from sweeps of the Mistral-7B shapes over M = 256..4096 on MI355X: the
   // eight-wave 256 x 256 kernel wins once its tile grid covers 9/16 of the CUs (W1/W3 from 512
   // rows, QKV from 1536, O and W2 from 2560); below that the 128-row LDS pipeline wins (it splits K
@@ -883,6 +891,11 @@ void gemm_choice(int epi, int M, int N, int K, int cus, int& stages, int& bk, in
 // stages of 64-deep ones on 128 or 256 rows (a forced eight-wave kernel with K % 64 != 0 lands there).
 void gemm_resolve(int epi, int M, int N, int K, int cus, int& stages, int& bk, int& bm) {
   gemm_choice(epi, M, N, K, cus, stages, bk, bm);
+  if (stages == 1) {
+    bk = kStreamK;
+    bm = (M + 31) / 32 * 32;
+    return;
+  }
   if (stages == 6 && K % 64 == 0) {
     bk = 64;
     bm = kBigM;
@@ -911,6 +924,32 @@ int launch_gemm(yhip_ctx* ctx, const GemmArgs& g, hipStream_t s) {
                                      g.P && g.sk_flags && g.abort_flag && g.p_floats >= (long)P * kSkSlotFloats);
     const unsigned epoch = sp.mains ? ++g_sk_epoch : 0;
     hipLaunchKernelGGL(gemm_pp_kernel<EPI>, dim3(sp.dp + sp.mains + sp.tails), dim3(512), 0, s, g, sp, epoch);
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return fail(ctx, YHIP_EDEVICE, std::string("gemm launch: ") + hipGetErrorString(e));
+    return YHIP_OK;
+  }
+  // Weight streaming: one workgroup per CU over (128-row weight blocks x K splits), as many splits as
+  // fit (a second workgroup per CU only adds partial sums: W2 at 32 rows 21.6 us with 8 splits, 24.0
+  // with 16; QKV 12.0 with 5, 14.8 with 10).
+  if (stages == 1) {
+    GemmArgs ga = g;
+    const long cus = ctx ? ctx->num_cus : device_cus();
+    const long tiles = (g.N + stream_cols(EPI) - 1) / stream_cols(EPI);
+    const long part_floats = (long)g.M * g.N * (EPI == kGemmSwiGLU ? 2 : 1);  // per split
+    const long ks = g.P ? std::min({cus / tiles, (long)(g.K / kStreamK), g.p_floats / part_floats}) : 1;
+    ga.ksplit = (int)std::max(1L, ks);
+    const dim3 grid(8 * (unsigned)((tiles * ga.ksplit + 7) / 8)), block(64 * kStreamWaves);
+    switch (bm) {
+      case 32: hipLaunchKernelGGL((gemm_stream_kernel<EPI, 32>), grid, block, 0, s, ga); break;
+      case 64: hipLaunchKernelGGL((gemm_stream_kernel<EPI, 64>), grid, block, 0, s, ga); break;
+      case 96: hipLaunchKernelGGL((gemm_stream_kernel<EPI, 96>), grid, block, 0, s, ga); break;
+      default: hipLaunchKernelGGL((gemm_stream_kernel<EPI, 128>), grid, block, 0, s, ga); break;
+    }
+    if (ga.ksplit > 1) {
+      const long total = (long)g.M * g.N;
+      hipLaunchKernelGGL(gemm_splitk_reduce<EPI>, dim3((unsigned)std::min<long>(4096, (total + 255) / 256)), dim3(256),
+                         0, s, ga);
+    }
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return fail(ctx, YHIP_EDEVICE, std::string("gemm launch: ") + hipGetErrorString(e));
     return YHIP_OK;

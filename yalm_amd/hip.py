@@ -278,7 +278,7 @@ def set_gemm_ksplit(n=0):
 def gemm_variant(M, N, K, mode):
     """(stages, k-step, workgroup rows) of the prefill GEMM yhip_prefill runs for this shape and mode
     under the current process-wide options (stages 6 = the eight-wave 256 x 256 kernel, 2..4 = the
-    LDS pipeline's depth)."""
+    LDS pipeline's depth, 1 = the weight-streaming kernel)."""
     out = [ctypes.c_int() for _ in range(3)]
     _check(lib().yhip_gemm_variant(M, N, K, mode, *[ctypes.byref(o) for o in out]))
     return tuple(o.value for o in out)
