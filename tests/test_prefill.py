@@ -239,6 +239,34 @@ def test_prefill_in_chunks_and_after_decode_steps():
     hm.close()
 
 
+@pytest.mark.parametrize("start,n", [(223, 5), (224, 5), (255, 33), (701, 1), (960, 64), (901, 90)])
+@pytest.mark.parametrize("shape", ["hd32_g1", "hd64_g2", "hd128_g4", "hd32_g8"])
+def test_prefill_key_split_behind_a_long_context(shape, start, n):
+    # Few queries behind a long cache: the keys are split over workgroups from two parts of four
+    # 32-key tiles on (224 cached positions), each part's sums merged by their maxima. Starts on and
+    # off the tile and split edges, one query, a full and a ragged query block, every count of query
+    # heads per kv head, against the oracle's steps from the same N(0, 1) cache. Weights of std 0.1
+    # make the attention a large part of every layer's output.
+    hd, g = {"hd32_g1": (32, 1), "hd64_g2": (64, 2), "hd128_g4": (128, 4), "hd32_g8": (32, 8)}[shape]
+    cfg = dict(MICRO, dim=256, hidden_dim=256, head_dim=hd, n_heads=2 * g, n_kv_heads=2, rotary_dim=hd,
+               max_seq_len=1024)
+    t = np_tensors(cfg, seed=71, std=0.1)
+    om = O.OracleModel(cfg, t)
+    hm = hip().HipModel(cfg, t)
+    rng = np.random.default_rng(start + n)
+    for layer in range(cfg["n_layers"]):
+        k, v = (f16(rng.standard_normal(cfg["n_kv_heads"] * hd * cfg["max_seq_len"])) for _ in range(2))
+        om.set_kv(layer, k, v)
+        hm.set_kv(layer, k, v)
+    toks = rng.integers(0, cfg["vocab_size"], n)
+    lh = hm.prefill(toks, start_pos=start)
+    lo = _sequential(om, toks, start=start)
+    assert npref.rel_l2(lh, lo) < PREFILL_LOGIT_TOL
+    _check_kv_close(om, hm, cfg["n_layers"], start + n)
+    om.close()
+    hm.close()
+
+
 def test_prefill_mistral_shape_two_layers():
     cfg = dict(TINY, dim=4096, hidden_dim=14336, head_dim=128, n_layers=2, n_heads=32, n_kv_heads=8,
                max_seq_len=512, rotary_dim=128)

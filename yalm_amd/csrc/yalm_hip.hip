@@ -995,18 +995,43 @@ int launch_gemm(yhip_ctx* ctx, const GemmArgs& g, hipStream_t s) {
   return YHIP_OK;
 }
 
+// Key splits of the prefill attention: a few queries behind a long context leave most CUs idle and
+// each workgroup a long chain of key tiles, so `splits` workgroups share the keys before them, as many
+// as fill the CUs once but with kSplitTiles tiles each at least: a part's start-up and its partial sums
+// cost about as much as four tiles (8 layers of the 7B shape, us per prefill of 16 tokens behind 1001 /
+// 3001 positions: unsplit 1267 / 1675, parts of at least 3 tiles 1130 / 1205, 4 1122 / 1195, 6 1150 /
+// 1191, 12 1194 / 1217; of 61 tokens 1456 / 1841, 1329 / 1372, 1313 / 1371, 1350 / 1375, 1382 / 1409).
+// No split where the partials would not fit the workspace.
+constexpr int kSplitTiles = 4;
+int prefill_attn_splits(const PrefillAttnArgs& p, int head_dim, int units, int cus, long p_floats) {
+  const long per = (long)p.n * p.n_heads * (head_dim + 2);  // floats per split
+  const long most = std::min({(long)(cus / units), (long)(p.start / 32 + 1) / kSplitTiles, p_floats / per});
+  return (int)std::max(1L, most);
+}
+
 // Workgroups of 64 * G * QT threads: G query heads x QT query tiles of 32 sharing each K/V tile.
+// ws: p_floats floats of scratch for the key splits' partials.
 template <int HD>
-bool launch_prefill_attn_hd(PrefillAttnArgs p, int G, int n_qtiles, hipStream_t s) {
-  auto go = [&](auto kernel, int qt, int threads) {
+bool launch_prefill_attn_hd(PrefillAttnArgs p, int G, int n_qtiles, float* ws, long p_floats, int cus, hipStream_t s) {
+  auto go = [&](auto kernel, auto split_kernel, int qt, int threads) {
     p.n_blocks = (n_qtiles + qt - 1) / qt;
-    hipLaunchKernelGGL(kernel, dim3(p.n_blocks * p.n_kv_heads), dim3(threads), 0, s, p);
+    const int units = p.n_blocks * p.n_kv_heads;
+    p.splits = prefill_attn_splits(p, HD, units, cus, p_floats);
+    if (p.splits == 1) {
+      hipLaunchKernelGGL(kernel, dim3(units), dim3(threads), 0, s, p);
+      return;
+    }
+    p.part_ml = (float2*)ws;
+    p.part_o = ws + 2L * p.splits * p.n * p.n_heads;
+    hipLaunchKernelGGL(split_kernel, dim3(units * p.splits), dim3(threads), 0, s, p);
+    hipLaunchKernelGGL(prefill_attn_merge_kernel, dim3(p.n, (p.n_heads * HD + 4 * kBlock - 1) / (4 * kBlock)),
+                       dim3(kBlock), 0, s, p, HD);
   };
   switch (G) {
-    case 1: go(prefill_attn_kernel<HD, 1, 4>, 4, 256); return true;
-    case 2: go(prefill_attn_kernel<HD, 2, 4>, 4, 512); return true;
-    case 4: go(prefill_attn_kernel<HD, 4, 2>, 2, 512); return true;
-    case 8: go(prefill_attn_kernel<HD, 8, 1>, 1, 512); return true;
+    case 1: go(prefill_attn_kernel<HD, 1, 4>, prefill_attn_kernel<HD, 1, 4, true>, 4, 256); return true;
+    case 2: go(prefill_attn_kernel<HD, 2, 4>, prefill_attn_kernel<HD, 2, 4, true>, 4, 512); return true;
+    case 4: go(prefill_attn_kernel<HD, 4, 2>, prefill_attn_kernel<HD, 4, 2, true>, 2, 512); return true;
+    case 8: go(prefill_attn_kernel<HD, 8, 1>, prefill_attn_kernel<HD, 8, 1, true>, 1, 512); return true;
     default: return false;
   }
 }
@@ -1103,9 +1128,9 @@ int run_prefill(yhip_ctx* ctx, const int* tokens, int n, int start, float* logit
     const int nqt = (n + 31) / 32;
     bool ok = false;
     switch (c.head_dim) {
-      case 32: ok = launch_prefill_attn_hd<32>(pa, G, nqt, s); break;
-      case 64: ok = launch_prefill_attn_hd<64>(pa, G, nqt, s); break;
-      case 128: ok = launch_prefill_attn_hd<128>(pa, G, nqt, s); break;
+      case 32: ok = launch_prefill_attn_hd<32>(pa, G, nqt, ctx->pf_P, ctx->pf_Pn, ctx->num_cus, s); break;
+      case 64: ok = launch_prefill_attn_hd<64>(pa, G, nqt, ctx->pf_P, ctx->pf_Pn, ctx->num_cus, s); break;
+      case 128: ok = launch_prefill_attn_hd<128>(pa, G, nqt, ctx->pf_P, ctx->pf_Pn, ctx->num_cus, s); break;
       default: break;
     }
     if (!ok) return fail(ctx, YHIP_EINVAL, "prefill: unsupported attention shape");
