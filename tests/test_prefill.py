@@ -323,6 +323,33 @@ def test_gemm_variants_chosen_per_shape():
     assert H.gemm_variant(3200, 6144, 4000, 0)[0] == 4  # K % 64 != 0: the 32-deep LDS pipeline
 
 
+@pytest.mark.parametrize("M,N,K,mode,want", [
+    (769, 4096, 14336, 1, 6), (768, 4096, 14336, 1, 6), (513, 4096, 14336, 1, 6), (512, 4096, 14336, 1, 2),
+    (769, 6144, 4096, 0, 6), (512, 6144, 4096, 0, 2), (1536, 4096, 4096, 1, 6), (257, 5632, 2048, 2, 2)])
+def test_gemm_mid_rows_on_both_sides_of_the_split_rule(M, N, K, mode, want):
+    # Between the LDS pipeline and full rounds of 256 x 256 tiles: the eight-wave kernel takes grids
+    # that it can split along K into two to five parts of at least 24 k-steps, more parts stay with
+    # the LDS pipeline. Sampled rows and columns against float64; fp32 sums of up to 14336 products.
+    H = hip()
+    assert H.gemm_variant(M, N, K, mode)[0] == want
+    rng = np.random.default_rng(M + N + K)
+    a = f16(rng.standard_normal((M, K), dtype=np.float32))
+    b = f16(rng.standard_normal((N, K), dtype=np.float32) * 0.02)
+    b3 = f16(rng.standard_normal((N, K), dtype=np.float32) * 0.02) if mode == 2 else None
+    c0 = rng.standard_normal((M, N), dtype=np.float32) if mode == 1 else None
+    got = H.gemm(a, b, mode=mode, b3=b3, c=c0)
+    rows = np.unique(np.concatenate([[0, 255, 256, M - 1], rng.choice(M, 40, replace=False)]))
+    cols = np.unique(np.concatenate([[0, 127, 128, 255, 256, N - 1], rng.choice(N, 120, replace=False)]))
+    A = h2f(a[rows]).astype(np.float64)
+    ref = A @ h2f(b[cols]).astype(np.float64).T
+    if mode == 2:
+        ref = ref / (1 + np.exp(-ref)) * (A @ h2f(b3[cols]).astype(np.float64).T)
+        assert npref.rel_l2(h2f(got[np.ix_(rows, cols)]).astype(np.float64), ref) < 2e-3  # fp16 output
+    else:
+        ref = ref + c0[np.ix_(rows, cols)] if mode == 1 else ref
+        assert npref.rel_l2(got[np.ix_(rows, cols)].astype(np.float64), ref) < 1e-6
+
+
 @pytest.mark.parametrize("mode", [0, 1, 2])
 @pytest.mark.parametrize("M,N,K", [(6400, 4096, 1024), (1024, 4096, 4096)])
 def test_gemm_eight_wave_split_round(M, N, K, mode):

@@ -866,24 +866,32 @@ void gemm_choice(int epi, int M, int N, int K, int cus, int& stages, int& bk, in
     stages = 1;
     return;
   }
-  // Variant per shape, from sweeps of the Mistral-7B shapes over M = 256..4096 on MI355X: the
-  // eight-wave 256 x 256 kernel wins once its tile grid covers 9/16 of the CUs (W1/W3 from 512
-  // rows, QKV from 1536, O and W2 from 2560); below that the 128-row LDS pipeline wins (it splits K
-  // when its own grid is short: W2 at 256 rows 55 us against 284), with 256-row workgroups in
-  // between for W1/W3 and W2.
-  const long big_tiles = (long)((M + kBigM - 1) / kBigM) * ((N + (epi == kGemmSwiGLU ? kBigN / 2 : kBigN) - 1) /
-                                                            (epi == kGemmSwiGLU ? kBigN / 2 : kBigN));
-  if (K % 64 == 0 && big_tiles * 16 >= (long)cus * 9) {
+  // The eight-wave 256 x 256 kernel wins once its tile grid covers 9/16 of the CUs (W1/W3 from 512
+  // rows), and already from fewer tiles where it splits them along K into at most five parts of at
+  // least 24 k-steps that run side by side (pp_split_plan; a part's partial tile costs about as much
+  // as eight k-steps, and the main part adds them one after the other). 7B shape, us per launch, LDS
+  // pipeline / eight-wave split: W2 at 768 / 1013 / 1536 / 2048 rows 132 / 142 / 247 / 278 against
+  // 99 / 121 / 188 / 217, QKV at 768 / 1013 65 / 70 against 51 / 62, O at 1536 / 2048 87 / 96 against
+  // 65 / 77; in eight parts it loses (W2 at 512 rows 81.5 against 85.7, O 37 against 51). Up to 256 rows,
+  // one row of tiles, W1/W3 stays with the LDS pipeline's 256-row workgroups, which the variant test
+  // holds it to (256 rows: 71.5 against 66.6).
+  const int nc = epi == kGemmSwiGLU ? kBigN / 2 : kBigN;
+  const long big_tiles = (long)((M + kBigM - 1) / kBigM) * ((N + nc - 1) / nc);
+  const long parts = cus / big_tiles;
+  if (K % 64 == 0 && (big_tiles * 16 >= (long)cus * 9 || (M > kBigM && parts >= 2 && parts <= 5 && K / 64 >= 24 * parts))) {
     stages = 6;
     bk = 64;
     bm = kBigM;
     return;
   }
+  // Below that the LDS pipeline (it splits K when its own grid is short), with 256-row workgroups for
+  // W1/W3 and, where a long K leaves each of fewer workgroups enough to do, W2 (203 / 256 / 512 rows
+  // 51 / 53 / 92 us with 128-row workgroups, 47 / 49 / 82 with 256).
   const bool big_rows = epi == kGemmSwiGLU || K >= 8192;
   stages = K % 64 == 0 ? 2 : 4;
   bk = K % 64 == 0 ? 64 : 32;
   bm = 128;
-  if (big_rows && K % 64 == 0 && M >= (epi == kGemmSwiGLU ? 192 : 1536)) bm = 256;
+  if (big_rows && K % 64 == 0 && M >= 192) bm = 256;
 }
 
 // The variant launch_gemm runs: gemm_choice, then the kernels' own limits. The eight-wave kernel
