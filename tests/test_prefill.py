@@ -267,6 +267,24 @@ def test_prefill_key_split_behind_a_long_context(shape, start, n):
     hm.close()
 
 
+@pytest.mark.parametrize("dim,n", [(96, 33), (4224, 2), (4224, 33), (8320, 5), (256, 1030)])
+def test_prefill_row_kernels_at_widths_off_their_blocks(dim, n):
+    # The kernels between the GEMMs: split partial sums + residual + norm (a row over 1024 threads of 4
+    # values: rows shorter than one pass, one value group past one and past two), q/k/v rows read
+    # from split partials, several workgroups to a row up to 1023 rows and one from there on.
+    cfg = dict(TINY, dim=dim, hidden_dim=256, n_heads=4, n_kv_heads=2, n_layers=2, vocab_size=512, max_seq_len=1056)
+    t = np_tensors(cfg, seed=73, std=0.03, gain="random")
+    om = O.OracleModel(cfg, t)
+    hm = hip().HipModel(cfg, t)
+    toks = np.random.default_rng(dim + n).integers(0, cfg["vocab_size"], n)
+    lh = hm.prefill(toks)
+    lo = _sequential(om, toks)
+    assert npref.rel_l2(lh, lo) < PREFILL_LOGIT_TOL
+    _check_kv_close(om, hm, cfg["n_layers"], n)
+    om.close()
+    hm.close()
+
+
 def test_prefill_mistral_shape_two_layers():
     cfg = dict(TINY, dim=4096, hidden_dim=14336, head_dim=128, n_layers=2, n_heads=32, n_kv_heads=8,
                max_seq_len=512, rotary_dim=128)

@@ -856,6 +856,58 @@ __global__ void __launch_bounds__(kBlock) rmsnorm_rows_kernel(const float* X, co
   for (int i = threadIdx.x; i < dim; i += kBlock) o[i] = __builtin_bit_cast(uint16_t, (f16)(x[i] * inv * gain[i]));
 }
 
+// The end of a residual GEMM whose K was split: X[t] += the sum of the split partials P [ksplit][n][dim] in
+// split order, and, with a gain, the next product's Xn[t] = fp16(rmsnorm(X[t])) in the same pass. One
+// launch and one trip of X instead of two, and 1024 threads to a row, so that all of a row's loads are
+// one round trip deep: 4.8 + 4.7 -> 4.7 us after
+// O and after W2 at 32 rows of the 7B shape, 6.5 + 4.8 -> 6.4 at 203 (256 threads to a row: 7.0 and 9.1).
+// dim % 4 == 0 and dim <= 16384 (prefill_supported, yhip_create).
+constexpr int kRowThreads = 1024;
+__global__ void __launch_bounds__(kRowThreads) splitk_resid_norm_kernel(const float* P, int ksplit, int n, float* X,
+                                                                        const float* gain, float eps, int dim,
+                                                                        uint16_t* Xn) {
+  __shared__ float red[kRowThreads / kWave];
+  constexpr int kMax4 = 4;  // float4 per thread
+  const int n4 = dim / 4;
+  f32x4* x4 = reinterpret_cast<f32x4*>(X + (long)blockIdx.x * dim);
+  const f32x4* p4 = reinterpret_cast<const f32x4*>(P + (long)blockIdx.x * dim);
+  const long step = (long)n * n4;
+  f32x4 v[kMax4], g[kMax4];
+  float ss = 0.f;
+#pragma unroll
+  for (int k = 0; k < kMax4; ++k) {
+    const int i = threadIdx.x + kRowThreads * k;
+    if (i >= n4) break;
+    const f32x4 x = x4[i];
+    if (gain) g[k] = reinterpret_cast<const f32x4*>(gain)[i];
+    v[k] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 8
+    for (int s = 0; s < ksplit; ++s) v[k] += p4[s * step + i];
+    v[k] += x;
+    x4[i] = v[k];
+    ss += v[k][0] * v[k][0] + v[k][1] * v[k][1] + v[k][2] * v[k][2] + v[k][3] * v[k][3];
+  }
+  if (!gain) return;
+  ss = wave_sum(ss);
+  if ((threadIdx.x & (kWave - 1)) == 0) red[threadIdx.x / kWave] = ss;
+  __syncthreads();
+  ss = 0.f;
+#pragma unroll
+  for (int w = 0; w < kRowThreads / kWave; ++w) ss += red[w];
+  const float inv = 1.0f / sqrtf(ss / (float)dim + eps);
+  unsigned long long* o = reinterpret_cast<unsigned long long*>(Xn + (long)blockIdx.x * dim);
+#pragma unroll
+  for (int k = 0; k < kMax4; ++k) {
+    const int i = threadIdx.x + kRowThreads * k;
+    if (i >= n4) break;
+    unsigned long long h = 0;
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      h |= (unsigned long long)__builtin_bit_cast(uint16_t, (f16)(v[k][e] * inv * g[k][e])) << (16 * e);
+    o[i] = h;
+  }
+}
+
 // Max over an aligned group of n lanes (n in {8, 16, 32}) by DPP moves inside the vector ALU (quad
 // permutes for xor 1 and 2, then the 8- and 16-lane mirrors, each pairing the two halves of the
 // previous group), plus one cross-row shuffle for 32; __shfl_xor took an LDS round trip per step.
@@ -873,43 +925,61 @@ __device__ __forceinline__ float group_max(float x, int n) {
   return x;
 }
 
+// The QKV GEMM's output: C [n][ldc], or, where the GEMM's K was split, the partials [ksplit][n][ldc],
+// summed in split order as they are read.
+struct QkvRowsArgs {
+  const float* C;
+  int ksplit;  // 1: C itself
+  int ldc, q_dim, kv_dim, head_dim, n;
+  float qkv_clip;
+  const float* inv_freq;
+  int start, msl;
+  uint16_t* Q;
+  float* qscale;
+  uint16_t* kcache;
+  uint16_t* vcache;
+  int q_blocks;  // workgroups per row on the q and k columns
+};
+__device__ __forceinline__ f32x4 qkv_sum4(const QkvRowsArgs& a, long at) {
+  const long step = (long)a.n * a.ldc;
+  f32x4 v = *reinterpret_cast<const f32x4*>(a.C + at);
+#pragma unroll 4
+  for (int s = 1; s < a.ksplit; ++s) v += *reinterpret_cast<const f32x4*>(a.C + s * step + at);
+  return v;
+}
+
 // Row t of the QKV GEMM output (position start + t): clip, RoPE on q and k pairs
 // (reference src/infer.cpp:197-215, 284-305), q as fp16 into Q, k as fp16 into the cache at the
-// row's position (no ring: start + n <= max_seq_len). The v columns go to v_rows_kernel.
+// row's position (no ring: start + n <= max_seq_len). The v columns go to v_rows.
 // Each query head of the row is stored scaled by the power of two that maps its largest |q| into
 // [2^14, 2^15) (q_range_exp), so any finite fp32 q fits fp16 with the same relative precision;
 // qscale[t][h] receives the inverse factor, which the attention applies to the head's scores.
-__global__ void __launch_bounds__(kBlock) qkv_rows_kernel(const float* C, int ldc, int q_dim, int kv_dim, int head_dim,
-                                                          float qkv_clip, const float* inv_freq, int start, int msl,
-                                                          uint16_t* Q, float* qscale, uint16_t* kcache) {
-  // (cos, sin) of pos * freq_k once per rotary pair k of the row, shared by all q and k heads
-  __shared__ float rope[128];  // head_dim <= 128 on the batched path (prefill_supported)
-  const int t = blockIdx.x, pos = start + t;
-  for (int k = threadIdx.x; k < head_dim / 2; k += kBlock) {
-    const float ang = (float)pos * inv_freq[k];
+__device__ __forceinline__ void qk_row(const QkvRowsArgs& a, int t, int part, float* rope) {
+  const int pos = a.start + t;
+  for (int k = threadIdx.x; k < a.head_dim / 2; k += kBlock) {
+    const float ang = (float)pos * a.inv_freq[k];
     rope[2 * k] = cosf(ang);
     rope[2 * k + 1] = sinf(ang);
   }
   __syncthreads();
-  const float* c = C + (long)t * ldc;
   // a lane takes 4 consecutive values (two rotary pairs): 16-byte loads, 8-byte stores (the 4 dims
   // lie in one 16-dim chunk of the K layout); a head is an aligned group of head_dim / 4 lanes
   // (a power of two, head_dim in {32, 64, 128}), and q_dim, kv_dim are multiples of 32
-  const int quads = (q_dim + kv_dim) / 4;  // q and k; v goes through v_rows_kernel
-  const int hq = head_dim / 4;
+  const int quads = (a.q_dim + a.kv_dim) / 4;
+  const int hq = a.head_dim / 4;
   // every thread runs the same number of iterations, so the head-wide maximum below can use
   // cross-lane shuffles; a head's group of lanes is all live or all dead
-  for (int p0 = 0; p0 < quads; p0 += kBlock) {
+  for (int p0 = part * kBlock; p0 < quads; p0 += a.q_blocks * kBlock) {
     const int p = p0 + threadIdx.x;
     const bool live = p < quads;
     const int i = 4 * p;
     f32x4 v = {0.f, 0.f, 0.f, 0.f};
     if (live) {
-      v = *reinterpret_cast<const f32x4*>(c + i);
-      const int j = i % head_dim;
+      v = qkv_sum4(a, (long)t * a.ldc + i);
+      const int j = i % a.head_dim;
 #pragma unroll
       for (int e = 0; e < 4; e += 2) {
-        const float v0 = clipf(v[e], qkv_clip), v1 = clipf(v[e + 1], qkv_clip);
+        const float v0 = clipf(v[e], a.qkv_clip), v1 = clipf(v[e + 1], a.qkv_clip);
         const float cs = rope[j + e], sn = rope[j + e + 1];
         v[e] = v0 * cs - v1 * sn;
         v[e + 1] = v0 * sn + v1 * cs;
@@ -917,22 +987,22 @@ __global__ void __launch_bounds__(kBlock) qkv_rows_kernel(const float* C, int ld
     }
     const float amax = group_max(fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3]))), hq);
     if (!live) continue;
-    if (i < q_dim) {
+    if (i < a.q_dim) {
       const int qe = q_range_exp(amax);
       const float qmul = __builtin_ldexpf(1.0f, qe);
 #pragma unroll
       for (int e = 0; e < 4; ++e) v[e] *= qmul;
-      if (p % hq == 0) qscale[(long)t * (q_dim / head_dim) + i / head_dim] = __builtin_ldexpf(1.0f, -qe);
+      if (p % hq == 0) a.qscale[(long)t * (a.q_dim / a.head_dim) + i / a.head_dim] = __builtin_ldexpf(1.0f, -qe);
     }
     unsigned long long h = 0;
 #pragma unroll
     for (int e = 0; e < 4; ++e) h |= (unsigned long long)__builtin_bit_cast(uint16_t, (f16)v[e]) << (16 * e);
-    if (i < q_dim) {
-      *reinterpret_cast<unsigned long long*>(Q + (long)t * q_dim + i) = h;
+    if (i < a.q_dim) {
+      *reinterpret_cast<unsigned long long*>(a.Q + (long)t * a.q_dim + i) = h;
     } else {  // k: dims j .. j+3 (j % 4 == 0) are adjacent in a 16-dim chunk of the K layout
-      const int ik = i - q_dim;
-      const int g = ik / head_dim, j = ik % head_dim;
-      *reinterpret_cast<unsigned long long*>(kcache + (long)g * head_dim * msl + k_cache_idx(j, pos, msl)) = h;
+      const int ik = i - a.q_dim;
+      const int g = ik / a.head_dim, j = ik % a.head_dim;
+      *reinterpret_cast<unsigned long long*>(a.kcache + (long)g * a.head_dim * a.msl + k_cache_idx(j, pos, a.msl)) = h;
     }
   }
 }
@@ -941,35 +1011,53 @@ __global__ void __launch_bounds__(kBlock) qkv_rows_kernel(const float* C, int ld
 // src/infer.cpp:284-305): V[g][d][pos] is position-contiguous, so a workgroup transposes a tile of
 // 64 positions x 64 value dims through LDS: 16-byte loads of 4 dims of a row, and, when the tile's
 // first position is a multiple of 8 and the tile is full, 16-byte stores of 8 positions of a dim
-// (otherwise 2-byte stores). kv_dim % 4 == 0.
-__global__ void __launch_bounds__(kBlock) v_rows_kernel(const float* C, int ldc, int q_dim, int kv_dim, int n,
-                                                        float qkv_clip, int start, int msl, uint16_t* vcache) {
-  __shared__ __attribute__((aligned(16))) uint16_t tile[64][64 + 8];  // [dim][position]
-  const int p0 = blockIdx.x * 64, d0 = blockIdx.y * 64;  // positions (rows of C), value dims
+// (otherwise 2-byte stores). The V cache of kv head g starts at (g * head_dim) * msl: one [kv_dim][msl]
+// matrix. kv_dim % 4 == 0.
+constexpr int kVTile = 64 + 8;  // LDS row of a value dim (halves), padded
+__device__ __forceinline__ void v_rows(const QkvRowsArgs& a, int p0, int d0, uint16_t (*tile)[kVTile]) {
   const int tid = threadIdx.x;
 #pragma unroll
   for (int k = 0; k < 4; ++k) {  // read: 16 lanes cover a row's 64 dims
     const int r = (tid >> 4) + 16 * k, d = d0 + 4 * (tid & 15), t = p0 + r;
     f32x4 v = {0.f, 0.f, 0.f, 0.f};
-    if (t < n && d < kv_dim) v = *reinterpret_cast<const f32x4*>(C + (long)t * ldc + q_dim + kv_dim + d);
+    if (t < a.n && d < a.kv_dim) v = qkv_sum4(a, (long)t * a.ldc + a.q_dim + a.kv_dim + d);
 #pragma unroll
-    for (int e = 0; e < 4; ++e) tile[4 * (tid & 15) + e][r] = __builtin_bit_cast(uint16_t, (f16)clipf(v[e], qkv_clip));
+    for (int e = 0; e < 4; ++e)
+      tile[4 * (tid & 15) + e][r] = __builtin_bit_cast(uint16_t, (f16)clipf(v[e], a.qkv_clip));
   }
   __syncthreads();
-  if ((start + p0) % 8 == 0 && p0 + 64 <= n) {
+  if ((a.start + p0) % 8 == 0 && p0 + 64 <= a.n) {
 #pragma unroll
     for (int k = 0; k < 2; ++k) {  // write: 8 lanes cover a dim's 64 positions
       const int r = (tid >> 3) + 32 * k, w = tid & 7, d = d0 + r;
-      if (d < kv_dim)
-        *reinterpret_cast<u32x4*>(vcache + (long)d * msl + start + p0 + 8 * w) =
+      if (d < a.kv_dim)
+        *reinterpret_cast<u32x4*>(a.vcache + (long)d * a.msl + a.start + p0 + 8 * w) =
             *reinterpret_cast<const u32x4*>(&tile[r][8 * w]);
     }
   } else {
     const int tx = tid & 63, ty = tid >> 6;
     for (int r = ty; r < 64; r += kBlock / 64) {  // write: a dim's 64 positions, coalesced
       const int d = d0 + r, t = p0 + tx;
-      if (t < n && d < kv_dim) vcache[(long)d * msl + start + t] = tile[r][tx];
+      if (t < a.n && d < a.kv_dim) a.vcache[(long)d * a.msl + a.start + t] = tile[r][tx];
     }
+  }
+}
+
+// Both parts in one launch: q_blocks workgroups per row, then one per 64 x 64 tile of v. Few rows take
+// several workgroups each (q_blocks), so that the launch is one memory round trip deep and not one per
+// 1024 columns: 32 rows of the 7B shape behind 5 K splits 4.8 + 5.9 + 4.8
+// us (reduce, q and k, v) -> 4.8, 3200 rows (no split) 22.4 + 5.5 -> 24.1.
+__global__ void __launch_bounds__(kBlock) qkv_rows_kernel(QkvRowsArgs a) {
+  __shared__ union {
+    float rope[128];  // (cos, sin) per rotary pair; head_dim <= 128 on the batched path (prefill_supported)
+    __attribute__((aligned(16))) uint16_t tile[64][kVTile];
+  } lds;
+  const int qk = a.n * a.q_blocks;
+  if ((int)blockIdx.x < qk) {
+    qk_row(a, blockIdx.x / a.q_blocks, blockIdx.x % a.q_blocks, lds.rope);
+  } else {
+    const int b = blockIdx.x - qk, pt = (a.n + 63) / 64;
+    v_rows(a, (b % pt) * 64, (b / pt) * 64, lds.tile);
   }
 }
 

@@ -918,10 +918,22 @@ void gemm_resolve(int epi, int M, int N, int K, int cus, int& stages, int& bk, i
   }
 }
 
+// The K splits of a GEMM: their partial sums reduced by a launch of its own, or (deferred not null) left
+// in g.P for the caller's next kernel, with their number in *deferred (1: the GEMM wrote its output).
+template <int EPI>
+void splitk_end(const GemmArgs& g, int* deferred, hipStream_t s) {
+  if (deferred) *deferred = std::max(1, g.ksplit);
+  if (g.ksplit <= 1 || deferred) return;
+  const long total = (long)g.M * g.N;
+  hipLaunchKernelGGL(gemm_splitk_reduce<EPI>, dim3((unsigned)std::min<long>(4096, (total + 255) / 256)), dim3(256), 0, s,
+                     g);
+}
+
 // Prefill GEMM launch. The variant is chosen per shape (gemm_choice) unless forced with the
 // process-wide options.
 template <int EPI>
-int launch_gemm(yhip_ctx* ctx, const GemmArgs& g, hipStream_t s) {
+int launch_gemm(yhip_ctx* ctx, const GemmArgs& g, hipStream_t s, int* deferred = nullptr) {
+  if (deferred) *deferred = 1;
   if (g.K % kGBK != 0 || g.M <= 0 || g.N <= 0) return fail(ctx, YHIP_EINVAL, "gemm: K must be a multiple of 32");
   int stages, bk, bm;
   gemm_resolve(EPI, g.M, g.N, g.K, ctx ? ctx->num_cus : device_cus(), stages, bk, bm);
@@ -953,11 +965,7 @@ int launch_gemm(yhip_ctx* ctx, const GemmArgs& g, hipStream_t s) {
       case 96: hipLaunchKernelGGL((gemm_stream_kernel<EPI, 96>), grid, block, 0, s, ga); break;
       default: hipLaunchKernelGGL((gemm_stream_kernel<EPI, 128>), grid, block, 0, s, ga); break;
     }
-    if (ga.ksplit > 1) {
-      const long total = (long)g.M * g.N;
-      hipLaunchKernelGGL(gemm_splitk_reduce<EPI>, dim3((unsigned)std::min<long>(4096, (total + 255) / 256)), dim3(256),
-                         0, s, ga);
-    }
+    splitk_end<EPI>(ga, deferred, s);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return fail(ctx, YHIP_EDEVICE, std::string("gemm launch: ") + hipGetErrorString(e));
     return YHIP_OK;
@@ -993,11 +1001,7 @@ int launch_gemm(yhip_ctx* ctx, const GemmArgs& g, hipStream_t s) {
     case 3 * 10000 + 8000 + 256: hipLaunchKernelGGL((gemm_lds_kernel<EPI, 3, 64, 256>), grid, dim3(512), 0, s, ga); break;
     default: return fail(ctx, YHIP_EINVAL, "gemm: no LDS-pipeline kernel for this variant");
   }
-  if (ga.ksplit > 1) {
-    const long total = (long)g.M * g.N;
-    hipLaunchKernelGGL(gemm_splitk_reduce<EPI>, dim3((unsigned)std::min<long>(4096, (total + 255) / 256)), dim3(256), 0,
-                       s, ga);
-  }
+  splitk_end<EPI>(ga, deferred, s);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return fail(ctx, YHIP_EDEVICE, std::string("gemm launch: ") + hipGetErrorString(e));
   return YHIP_OK;
@@ -1095,11 +1099,22 @@ int run_prefill(yhip_ctx* ctx, const int* tokens, int n, int start, float* logit
   HIP_TRY(ctx, hipMemcpyAsync(ctx->pf_tok, tokens, (size_t)n * sizeof(int), hipMemcpyHostToDevice, s));
   hipLaunchKernelGGL(embed_rows_kernel, dim3(n), dim3(kBlock), 0, s, (const uint16_t*)ctx->embed,
                      (const int*)ctx->pf_tok, ctx->pf_X, c.dim);
+  auto norm_rows = [&](const float* gain) {
+    hipLaunchKernelGGL(rmsnorm_rows_kernel, dim3(n), dim3(kBlock), 0, s, (const float*)ctx->pf_X, gain, c.norm_eps,
+                       c.dim, ctx->pf_Xn);
+  };
+  // a residual GEMM's K splits into X, and the norm of X that the next product reads (gain null: none)
+  auto resid_norm = [&](int splits, const float* gain) {
+    if (splits > 1)
+      hipLaunchKernelGGL(splitk_resid_norm_kernel, dim3(n), dim3(kRowThreads), 0, s, (const float*)ctx->pf_P, splits, n,
+                         ctx->pf_X, gain, c.norm_eps, c.dim, ctx->pf_Xn);
+    else if (gain)
+      norm_rows(gain);
+  };
+  if (c.n_layers > 0) norm_rows(ctx->layers[0].rms_att);
   for (int l = 0; l < c.n_layers; ++l) {
     const LayerW& L = ctx->layers[l];
-    int rc;
-    hipLaunchKernelGGL(rmsnorm_rows_kernel, dim3(n), dim3(kBlock), 0, s, (const float*)ctx->pf_X,
-                       (const float*)L.rms_att, c.norm_eps, c.dim, ctx->pf_Xn);
+    int rc, splits;
     GemmArgs g;
     memset(&g, 0, sizeof(g));
     g.A = ctx->pf_Xn;
@@ -1115,13 +1130,26 @@ int run_prefill(yhip_ctx* ctx, const int* tokens, int n, int start, float* logit
     g.p_floats = ctx->pf_Pn;
     g.sk_flags = ctx->pf_flags;
     g.abort_flag = ctx->step_abort;
-    if ((rc = launch_gemm<kGemmStore>(ctx, g, s))) return rc;
-    hipLaunchKernelGGL(qkv_rows_kernel, dim3(n), dim3(kBlock), 0, s, (const float*)ctx->pf_C, qd + 2 * kvd, qd, kvd,
-                       c.head_dim, c.qkv_clip, (const float*)ctx->inv_freq, start, c.max_seq_len, ctx->pf_Q,
-                       ctx->pf_qs, ctx->kcache(l));
-    // the V cache of kv head g at (g * head_dim + d) * msl: one [kv_dim][msl] matrix
-    hipLaunchKernelGGL(v_rows_kernel, dim3((n + 63) / 64, (kvd + 63) / 64), dim3(kBlock), 0, s, (const float*)ctx->pf_C,
-                       qd + 2 * kvd, qd, kvd, n, c.qkv_clip, start, c.max_seq_len, ctx->vcache(l));
+    if ((rc = launch_gemm<kGemmStore>(ctx, g, s, &splits))) return rc;
+    QkvRowsArgs qa;
+    qa.C = splits > 1 ? ctx->pf_P : ctx->pf_C;
+    qa.ksplit = splits;
+    qa.ldc = qd + 2 * kvd;
+    qa.q_dim = qd;
+    qa.kv_dim = kvd;
+    qa.head_dim = c.head_dim;
+    qa.n = n;
+    qa.qkv_clip = c.qkv_clip;
+    qa.inv_freq = ctx->inv_freq;
+    qa.start = start;
+    qa.msl = c.max_seq_len;
+    qa.Q = ctx->pf_Q;
+    qa.qscale = ctx->pf_qs;
+    qa.kcache = ctx->kcache(l);
+    qa.vcache = ctx->vcache(l);
+    // from 4 rows per CU on a workgroup per row fills the GPU, and shares the row's RoPE table
+    qa.q_blocks = n >= 4 * ctx->num_cus ? 1 : ((qd + kvd) / 4 + kBlock - 1) / kBlock;
+    hipLaunchKernelGGL(qkv_rows_kernel, dim3(n * qa.q_blocks + (n + 63) / 64 * ((kvd + 63) / 64)), dim3(kBlock), 0, s, qa);
     PrefillAttnArgs pa;
     pa.Q = ctx->pf_Q;
     pa.qscale = ctx->pf_qs;
@@ -1156,9 +1184,8 @@ int run_prefill(yhip_ctx* ctx, const int* tokens, int n, int start, float* logit
     g.p_floats = ctx->pf_Pn;
     g.sk_flags = ctx->pf_flags;
     g.abort_flag = ctx->step_abort;
-    if ((rc = launch_gemm<kGemmResid>(ctx, g, s))) return rc;
-    hipLaunchKernelGGL(rmsnorm_rows_kernel, dim3(n), dim3(kBlock), 0, s, (const float*)ctx->pf_X,
-                       (const float*)L.rms_ffn, c.norm_eps, c.dim, ctx->pf_Xn);
+    if ((rc = launch_gemm<kGemmResid>(ctx, g, s, &splits))) return rc;
+    resid_norm(splits, L.rms_ffn);
     memset(&g, 0, sizeof(g));
     g.A = ctx->pf_Xn;
     g.lda = c.dim;
@@ -1190,7 +1217,8 @@ int run_prefill(yhip_ctx* ctx, const int* tokens, int n, int start, float* logit
     g.p_floats = ctx->pf_Pn;
     g.sk_flags = ctx->pf_flags;
     g.abort_flag = ctx->step_abort;
-    if ((rc = launch_gemm<kGemmResid>(ctx, g, s))) return rc;
+    if ((rc = launch_gemm<kGemmResid>(ctx, g, s, &splits))) return rc;
+    resid_norm(splits, l + 1 < c.n_layers ? ctx->layers[l + 1].rms_att : nullptr);
   }
   HIP_TRY(ctx, hipGetLastError());
   // a timed-out wait of a split-last-round GEMM, checked after the next synchronisation
