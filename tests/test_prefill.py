@@ -343,11 +343,14 @@ def test_gemm_variants_chosen_per_shape():
 
 @pytest.mark.parametrize("M,N,K,mode,want", [
     (769, 4096, 14336, 1, 6), (768, 4096, 14336, 1, 6), (513, 4096, 14336, 1, 6), (512, 4096, 14336, 1, 2),
-    (769, 6144, 4096, 0, 6), (512, 6144, 4096, 0, 2), (1536, 4096, 4096, 1, 6), (257, 5632, 2048, 2, 2)])
+    (769, 6144, 4096, 0, 6), (640, 6144, 4096, 0, 2), (1025, 4096, 4096, 1, 6), (700, 4100, 4096, 1, 2),
+    (257, 5632, 2048, 2, 2), (203, 1030, 5504, 1, 2), (203, 516, 5504, 0, 2), (150, 520, 4160, 2, 2)])
 def test_gemm_mid_rows_on_both_sides_of_the_split_rule(M, N, K, mode, want):
     # Between the LDS pipeline and full rounds of 256 x 256 tiles: the eight-wave kernel takes grids
-    # that it can split along K into two to five parts of at least 24 k-steps, more parts stay with
-    # the LDS pipeline. Sampled rows and columns against float64; fp32 sums of up to 14336 products.
+    # that it can split along K into two to five parts of at least 20 k-steps where 128-row tiles need
+    # a second round or K is long, the rest stays with the LDS pipeline; there unsplit with a residual
+    # at ragged row and column tiles (700 x 4100), and split into parts that do not divide the k-steps
+    # (5504 / 64 = 86 over 14 and 25 parts, 4160 / 64 = 65 over 14). Sampled rows and columns against float64; fp32 sums of up to 14336 products.
     H = hip()
     assert H.gemm_variant(M, N, K, mode)[0] == want
     rng = np.random.default_rng(M + N + K)
@@ -356,7 +359,7 @@ def test_gemm_mid_rows_on_both_sides_of_the_split_rule(M, N, K, mode, want):
     b3 = f16(rng.standard_normal((N, K), dtype=np.float32) * 0.02) if mode == 2 else None
     c0 = rng.standard_normal((M, N), dtype=np.float32) if mode == 1 else None
     got = H.gemm(a, b, mode=mode, b3=b3, c=c0)
-    rows = np.unique(np.concatenate([[0, 255, 256, M - 1], rng.choice(M, 40, replace=False)]))
+    rows = np.unique(np.concatenate([[0, 127, 128, min(255, M - 1), min(256, M - 1), M - 1], rng.choice(M, 40, replace=False)]))
     cols = np.unique(np.concatenate([[0, 127, 128, 255, 256, N - 1], rng.choice(N, 120, replace=False)]))
     A = h2f(a[rows]).astype(np.float64)
     ref = A @ h2f(b[cols]).astype(np.float64).T

@@ -868,17 +868,21 @@ void gemm_choice(int epi, int M, int N, int K, int cus, int& stages, int& bk, in
   }
   // The eight-wave 256 x 256 kernel wins once its tile grid covers 9/16 of the CUs (W1/W3 from 512
   // rows), and already from fewer tiles where it splits them along K into at most five parts of at
-  // least 24 k-steps that run side by side (pp_split_plan; a part's partial tile costs about as much
-  // as eight k-steps, and the main part adds them one after the other). 7B shape, us per launch, LDS
-  // pipeline / eight-wave split: W2 at 768 / 1013 / 1536 / 2048 rows 132 / 142 / 247 / 278 against
-  // 99 / 121 / 188 / 217, QKV at 768 / 1013 65 / 70 against 51 / 62, O at 1536 / 2048 87 / 96 against
-  // 65 / 77; in eight parts it loses (W2 at 512 rows 81.5 against 85.7, O 37 against 51). Up to 256 rows,
-  // one row of tiles, W1/W3 stays with the LDS pipeline's 256-row workgroups, which the variant test
-  // holds it to (256 rows: 71.5 against 66.6).
+  // least 20 k-steps that run side by side (pp_split_plan; a part's partial tile costs about as much
+  // as eight k-steps, and the main part adds them one after the other) and the LDS pipeline would
+  // need a second round of 128-row tiles or has a long K to walk in one. 7B shape, us per launch, LDS
+  // pipeline / eight-wave split: W2 at 640 / 768 / 1013 / 1536 / 2048 rows 136 / 137 / 151 / 249 /
+  // 281 against 106 / 107 / 129 / 199 / 225, QKV at 768 / 1013 64 / 70 against 55 / 64, O at 1280 /
+  // 1536 69 / 72 against 62 / 68; and where the LDS pipeline's one round holds it wins: QKV at 512 /
+  // 640 46 / 48 against 49 / 54, O at 640 / 1013 46 / 51 against 51 / 56; so it does against eight
+  // parts (W2 at 512 rows 83 against 88). Up to 256 rows, one row of tiles, W1/W3 stays with the LDS
+  // pipeline's 256-row workgroups, which the variant test holds it to (256 rows: 71.5 against 66.6).
   const int nc = epi == kGemmSwiGLU ? kBigN / 2 : kBigN;
   const long big_tiles = (long)((M + kBigM - 1) / kBigM) * ((N + nc - 1) / nc);
+  const long tiles = (long)((M + kGBM - 1) / kGBM) * ((N + nc / 2 - 1) / (nc / 2));
   const long parts = cus / big_tiles;
-  if (K % 64 == 0 && (big_tiles * 16 >= (long)cus * 9 || (M > kBigM && parts >= 2 && parts <= 5 && K / 64 >= 24 * parts))) {
+  const bool split_parts = M > kBigM && parts >= 2 && parts <= 5 && K / 64 >= 20 * parts && (K >= 8192 || tiles > cus);
+  if (K % 64 == 0 && (big_tiles * 16 >= (long)cus * 9 || split_parts)) {
     stages = 6;
     bk = 64;
     bm = kBigM;
@@ -971,9 +975,11 @@ int launch_gemm(yhip_ctx* ctx, const GemmArgs& g, hipStream_t s, int* deferred =
     return YHIP_OK;
   }
   const int ncols = EPI == kGemmSwiGLU ? kGBN / 2 : kGBN;
-  // Split-K when the output has too few tiles to fill the GPU (short prompts): the largest power of
-  // two that keeps tiles x splits within one workgroup per CU, divides the k-steps and leaves each
-  // split at least two of them; the partials go to the caller's workspace (none: no split).
+  // Split-K when the output has too few tiles to fill the GPU (short prompts): as many splits as keep
+  // tiles x splits within one workgroup per CU and leave each split at least two k-steps (spans differ
+  // by one k-step where they do not divide: W2 4096 x 11008 at 203 rows in 4 splits, the largest power
+  // of two that divides its 172 k-steps, 55.4 us, in 8 40.6); the partials go to the caller's
+  // workspace (none: no split).
   GemmArgs ga = g;
   ga.ksplit = 1;
   const long tiles = (long)((g.M + bm - 1) / bm) * ((g.N + ncols - 1) / ncols);
@@ -985,9 +991,7 @@ int launch_gemm(yhip_ctx* ctx, const GemmArgs& g, hipStream_t s, int* deferred =
       if (ksteps % ga.ksplit != 0) return fail(ctx, YHIP_EINVAL, "gemm_ksplit must divide the k-steps");
     } else {
       const long cus = ctx ? ctx->num_cus : device_cus();
-      while (tiles * ga.ksplit * 2 <= cus && ksteps % (ga.ksplit * 2) == 0 && ksteps / (ga.ksplit * 2) >= 2 &&
-             part_floats * ga.ksplit * 2 <= g.p_floats)
-        ga.ksplit *= 2;
+      ga.ksplit = (int)std::max(1L, std::min({cus / tiles, (long)ksteps / 2, g.p_floats / part_floats}));
     }
     if (ga.ksplit > 1 && part_floats * ga.ksplit > g.p_floats)
       return fail(ctx, YHIP_EINVAL, "gemm: split-K workspace too small");
