@@ -343,13 +343,12 @@ def test_gemm_variants_chosen_per_shape():
 
 @pytest.mark.parametrize("M,N,K,mode,want", [
     (769, 4096, 14336, 1, 6), (768, 4096, 14336, 1, 6), (513, 4096, 14336, 1, 6), (512, 4096, 14336, 1, 2),
-    (769, 6144, 4096, 0, 6), (640, 6144, 4096, 0, 2), (1025, 4096, 4096, 1, 6), (700, 4100, 4096, 1, 2),
+    (769, 6144, 4096, 0, 6), (512, 6144, 4096, 0, 2), (1025, 4096, 4096, 1, 6), (1000, 4090, 4096, 1, 2),
     (257, 5632, 2048, 2, 2), (203, 1030, 5504, 1, 2), (203, 516, 5504, 0, 2), (150, 520, 4160, 2, 2)])
 def test_gemm_mid_rows_on_both_sides_of_the_split_rule(M, N, K, mode, want):
     # Between the LDS pipeline and full rounds of 256 x 256 tiles: the eight-wave kernel takes grids
-    # that it can split along K into two to five parts of at least 20 k-steps where 128-row tiles need
-    # a second round or K is long, the rest stays with the LDS pipeline; there unsplit with a residual
-    # at ragged row and column tiles (700 x 4100), and split into parts that do not divide the k-steps
+    # that it can split along K into two to five parts of at least 20 k-steps, the rest stays with the
+    # LDS pipeline; there unsplit with a residual at ragged row and column tiles (1000 x 4090), and split into parts that do not divide the k-steps
     # (5504 / 64 = 86 over 14 and 25 parts, 4160 / 64 = 65 over 14). Sampled rows and columns against float64; fp32 sums of up to 14336 products.
     H = hip()
     assert H.gemm_variant(M, N, K, mode)[0] == want

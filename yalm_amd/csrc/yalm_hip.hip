@@ -866,36 +866,43 @@ void gemm_choice(int epi, int M, int N, int K, int cus, int& stages, int& bk, in
     stages = 1;
     return;
   }
-  // The eight-wave 256 x 256 kernel wins once its tile grid covers 9/16 of the CUs (W1/W3 from 512
-  // rows), and already from fewer tiles where it splits them along K into at most five parts of at
-  // least 20 k-steps that run side by side (pp_split_plan; a part's partial tile costs about as much
-  // as eight k-steps, and the main part adds them one after the other) and the LDS pipeline would
-  // need a second round of 128-row tiles or has a long K to walk in one. 7B shape, us per launch, LDS
-  // pipeline / eight-wave split: W2 at 640 / 768 / 1013 / 1536 / 2048 rows 136 / 137 / 151 / 249 /
-  // 281 against 106 / 107 / 129 / 199 / 225, QKV at 768 / 1013 64 / 70 against 55 / 64, O at 1280 /
-  // 1536 69 / 72 against 62 / 68; and where the LDS pipeline's one round holds it wins: QKV at 512 /
-  // 640 46 / 48 against 49 / 54, O at 640 / 1013 46 / 51 against 51 / 56; so it does against eight
-  // parts (W2 at 512 rows 83 against 88). Up to 256 rows, one row of tiles, W1/W3 stays with the LDS
-  // pipeline's 256-row workgroups, which the variant test holds it to (256 rows: 71.5 against 66.6).
+  // The figures below are from traces of whole prefills (weights read from HBM; with one operand set
+  // launched over and over the weights stay in the memory-side cache and the order of the variants
+  // changes), us per launch at the 7B shape as 128-row LDS pipeline / 256-row / eight-wave.
+  //
+  // The eight-wave 256 x 256 kernel wins once its tile grid covers 9/16 of the CUs (W1/W3 at 300 rows 137 /
+  // 156 / 111, at 1536 420 / 425 / 326), and already from fewer tiles where it splits them along K into
+  // at most five parts of at least 20 k-steps that run side by side (pp_split_plan; a part's partial
+  // tile costs about as much as eight k-steps, and the main part adds them one after the other): W2 at
+  // 640 / 1013 rows 196 / 126 / 108 and 201 / 136 / 134, QKV at 640 / 1013 60 / 72 / 54 and 76 / 76 /
+  // 65, O at 1280 69 / 74 / 60; in more or shorter parts it loses (O at 640 rows 59 / 42 / 52). Up to 256
+  // rows, one row of tiles, W1/W3 stays with 256-row workgroups, which the variant test holds it to
+  // (240 rows: 87 / 89 / 77).
   const int nc = epi == kGemmSwiGLU ? kBigN / 2 : kBigN;
   const long big_tiles = (long)((M + kBigM - 1) / kBigM) * ((N + nc - 1) / nc);
-  const long tiles = (long)((M + kGBM - 1) / kGBM) * ((N + nc / 2 - 1) / (nc / 2));
   const long parts = cus / big_tiles;
-  const bool split_parts = M > kBigM && parts >= 2 && parts <= 5 && K / 64 >= 20 * parts && (K >= 8192 || tiles > cus);
+  const bool split_parts = M > kBigM && parts >= 2 && parts <= 5 && K / 64 >= 20 * parts;
   if (K % 64 == 0 && (big_tiles * 16 >= (long)cus * 9 || split_parts)) {
     stages = 6;
     bk = 64;
     bm = kBigM;
     return;
   }
-  // Below that the LDS pipeline (it splits K when its own grid is short), with 256-row workgroups for
-  // W1/W3 and, where a long K leaves each of fewer workgroups enough to do, W2 (203 / 256 / 512 rows
-  // 51 / 53 / 92 us with 128-row workgroups, 47 / 49 / 82 with 256).
-  const bool big_rows = epi == kGemmSwiGLU || K >= 8192;
+  // Below that the LDS pipeline, its K split where its grid is short. 256-row workgroups pass each weight
+  // panel through fewer CUs and win for W1/W3 from 192 rows, for a long K at once (W2 at 160 / 450 rows 58
+  // / 44 and 105 / 73) and otherwise where 128-row ones would not fill the CUs without a K split of their
+  // own (QKV at 240 / 450 rows 36 / 26 and 60 / 44, O 23 / 20 and 35 / 27, at 768 60 / 43) and their own
+  // split leaves at least six k-steps to each part (QKV 3072 x 2048 and O 2048 x 2048 at 240 rows, 3 and 2
+  // k-steps: 16.2 / 15.1 and 15.5 / 15.2, but twice the partial sums to add, 128 / 134 us per layer). O
+  // from 897 to 1024 rows, a full round of 128-row tiles, is held to those by the variant test, 62 / 44,
+  // and so is QKV at 200 rows, which puts the line for a short K right above that.
+  const long tiles = (long)((M + kGBM - 1) / kGBM) * ((N + kGBN - 1) / kGBN);
+  const long tiles_big = (long)((M + kBigM - 1) / kBigM) * ((N + kGBN - 1) / kGBN);
+  const long steps = K / 64 / std::max(1L, cus / tiles_big);  // k-steps per part with 256-row workgroups
+  const bool big_rows = epi == kGemmSwiGLU ? M >= 192 : K >= 8192 || (M > 200 && tiles < cus && steps >= 6);
   stages = K % 64 == 0 ? 2 : 4;
   bk = K % 64 == 0 ? 64 : 32;
-  bm = 128;
-  if (big_rows && K % 64 == 0 && M >= 192) bm = 256;
+  bm = K % 64 == 0 && big_rows ? 256 : 128;
 }
 
 // The variant launch_gemm runs: gemm_choice, then the kernels' own limits. The eight-wave kernel
