@@ -285,6 +285,30 @@ def test_prefill_row_kernels_at_widths_off_their_blocks(dim, n):
     hm.close()
 
 
+@pytest.mark.parametrize("n_layers", [1, 2])
+@pytest.mark.parametrize("start,n", [(0, 1), (0, 2), (0, 130), (300, 33), (300, 1)])
+def test_prefill_last_layer_runs_the_last_row(n_layers, start, n):
+    # Behind the last layer's K/V only the last row goes on (no row without logits): logits, caches, and
+    # a decode step behind each, with the last layer also the first, one row, the last row alone in
+    # its query tile (33, 130 = 4 * 32 + 2) and behind a cache long enough for the key split.
+    cfg = dict(TINY, n_layers=n_layers, vocab_size=512)
+    t = np_tensors(cfg, seed=75, std=0.1)
+    om = O.OracleModel(cfg, t)
+    toks = np.random.default_rng(start + n).integers(0, cfg["vocab_size"], start + n + 1)
+    lo = _sequential(om, toks[:-1])
+    nxt = om.forward(int(toks[-1]), start + n)
+    for logits in (True, False):
+        hm = hip().HipModel(cfg, t)
+        if start:
+            hm.prefill(toks[:start], logits=False)
+        lh = hm.prefill(toks[start:-1], start_pos=start, logits=logits)
+        assert lh is None if not logits else npref.rel_l2(lh, lo) < PREFILL_LOGIT_TOL
+        assert npref.rel_l2(hm.forward(int(toks[-1]), start + n), nxt) < PREFILL_LOGIT_TOL
+        _check_kv_close(om, hm, n_layers, start + n + 1)
+        hm.close()
+    om.close()
+
+
 def test_prefill_mistral_shape_two_layers():
     cfg = dict(TINY, dim=4096, hidden_dim=14336, head_dim=128, n_layers=2, n_heads=32, n_kv_heads=8,
                max_seq_len=512, rotary_dim=128)

@@ -1110,19 +1110,19 @@ int run_prefill(yhip_ctx* ctx, const int* tokens, int n, int start, float* logit
   HIP_TRY(ctx, hipMemcpyAsync(ctx->pf_tok, tokens, (size_t)n * sizeof(int), hipMemcpyHostToDevice, s));
   hipLaunchKernelGGL(embed_rows_kernel, dim3(n), dim3(kBlock), 0, s, (const uint16_t*)ctx->embed,
                      (const int*)ctx->pf_tok, ctx->pf_X, c.dim);
-  auto norm_rows = [&](const float* gain) {
-    hipLaunchKernelGGL(rmsnorm_rows_kernel, dim3(n), dim3(kBlock), 0, s, (const float*)ctx->pf_X, gain, c.norm_eps,
-                       c.dim, ctx->pf_Xn);
+  auto norm_rows = [&](int rows, const float* X, const float* gain) {
+    hipLaunchKernelGGL(rmsnorm_rows_kernel, dim3(rows), dim3(kBlock), 0, s, X, gain, c.norm_eps, c.dim, ctx->pf_Xn);
   };
   // a residual GEMM's K splits into X, and the norm of X that the next product reads (gain null: none)
-  auto resid_norm = [&](int splits, const float* gain) {
+  auto resid_norm = [&](int splits, int rows, float* X, const float* gain) {
     if (splits > 1)
-      hipLaunchKernelGGL(splitk_resid_norm_kernel, dim3(n), dim3(kRowThreads), 0, s, (const float*)ctx->pf_P, splits, n,
-                         ctx->pf_X, gain, c.norm_eps, c.dim, ctx->pf_Xn);
+      hipLaunchKernelGGL(splitk_resid_norm_kernel, dim3(rows), dim3(kRowThreads), 0, s, (const float*)ctx->pf_P, splits,
+                         rows, X, gain, c.norm_eps, c.dim, ctx->pf_Xn);
     else if (gain)
-      norm_rows(gain);
+      norm_rows(rows, X, gain);
   };
-  if (c.n_layers > 0) norm_rows(ctx->layers[0].rms_att);
+  int first = 0;  // first row that what follows still needs
+  if (c.n_layers > 0) norm_rows(n, ctx->pf_X, ctx->layers[0].rms_att);
   for (int l = 0; l < c.n_layers; ++l) {
     const LayerW& L = ctx->layers[l];
     int rc, splits;
@@ -1161,18 +1161,27 @@ int run_prefill(yhip_ctx* ctx, const int* tokens, int n, int start, float* logit
     // from 4 rows per CU on a workgroup per row fills the GPU, and shares the row's RoPE table
     qa.q_blocks = n >= 4 * ctx->num_cus ? 1 : ((qd + kvd) / 4 + kBlock - 1) / kBlock;
     hipLaunchKernelGGL(qkv_rows_kernel, dim3(n * qa.q_blocks + (n + 63) / 64 * ((kvd + 63) / 64)), dim3(kBlock), 0, s, qa);
+    // Behind the last layer's K and V only the last row is read (by the lm_head), and without logits
+    // nothing is: its attention, O and FFN run for that row alone, 3% of a 32-layer prefill of 3200
+    // tokens (46.9 -> 45.8 ms).
+    if (l + 1 == c.n_layers) {
+      if (!logits_host) break;
+      first = n - 1;
+    }
+    const int m = n - first;  // rows from here on
+    float* X = ctx->pf_X + (size_t)first * c.dim;
     PrefillAttnArgs pa;
-    pa.Q = ctx->pf_Q;
-    pa.qscale = ctx->pf_qs;
+    pa.Q = ctx->pf_Q + (size_t)first * qd;
+    pa.qscale = ctx->pf_qs + (size_t)first * c.n_heads;
     pa.kcache = ctx->kcache(l);
     pa.vcache = ctx->vcache(l);
     pa.out = ctx->pf_A;
-    pa.n = n;
-    pa.start = start;
+    pa.n = m;
+    pa.start = start + first;
     pa.msl = c.max_seq_len;
     pa.n_heads = c.n_heads;
     pa.n_kv_heads = c.n_kv_heads;
-    const int nqt = (n + 31) / 32;
+    const int nqt = (m + 31) / 32;
     bool ok = false;
     switch (c.head_dim) {
       case 32: ok = launch_prefill_attn_hd<32>(pa, G, nqt, ctx->pf_P, ctx->pf_Pn, ctx->num_cus, s); break;
@@ -1186,9 +1195,9 @@ int run_prefill(yhip_ctx* ctx, const int* tokens, int n, int start, float* logit
     g.lda = qd;
     g.B = L.wo;
     g.ldb = qd;
-    g.C = ctx->pf_X;
+    g.C = X;
     g.ldc = c.dim;
-    g.M = n;
+    g.M = m;
     g.N = c.dim;
     g.K = qd;
     g.P = ctx->pf_P;
@@ -1196,7 +1205,7 @@ int run_prefill(yhip_ctx* ctx, const int* tokens, int n, int start, float* logit
     g.sk_flags = ctx->pf_flags;
     g.abort_flag = ctx->step_abort;
     if ((rc = launch_gemm<kGemmResid>(ctx, g, s, &splits))) return rc;
-    resid_norm(splits, L.rms_ffn);
+    resid_norm(splits, m, X, L.rms_ffn);
     memset(&g, 0, sizeof(g));
     g.A = ctx->pf_Xn;
     g.lda = c.dim;
@@ -1205,7 +1214,7 @@ int run_prefill(yhip_ctx* ctx, const int* tokens, int n, int start, float* logit
     g.ldb = c.dim;
     g.H = ctx->pf_H;
     g.ldh = c.hidden_dim;
-    g.M = n;
+    g.M = m;
     g.N = c.hidden_dim;
     g.K = c.dim;
     g.act = c.act;
@@ -1219,9 +1228,9 @@ int run_prefill(yhip_ctx* ctx, const int* tokens, int n, int start, float* logit
     g.lda = c.hidden_dim;
     g.B = L.w2;
     g.ldb = c.hidden_dim;
-    g.C = ctx->pf_X;
+    g.C = X;
     g.ldc = c.dim;
-    g.M = n;
+    g.M = m;
     g.N = c.dim;
     g.K = c.hidden_dim;
     g.P = ctx->pf_P;
@@ -1229,7 +1238,7 @@ int run_prefill(yhip_ctx* ctx, const int* tokens, int n, int start, float* logit
     g.sk_flags = ctx->pf_flags;
     g.abort_flag = ctx->step_abort;
     if ((rc = launch_gemm<kGemmResid>(ctx, g, s, &splits))) return rc;
-    resid_norm(splits, l + 1 < c.n_layers ? ctx->layers[l + 1].rms_att : nullptr);
+    resid_norm(splits, m, X, l + 1 < c.n_layers ? ctx->layers[l + 1].rms_att : nullptr);
   }
   HIP_TRY(ctx, hipGetLastError());
   // a timed-out wait of a split-last-round GEMM, checked after the next synchronisation
