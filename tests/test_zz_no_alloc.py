@@ -104,3 +104,19 @@ def test_noalloc_attention_rejects_sizes_beyond_its_scratch():
         rc = H.lib().yhip_attention_noalloc(dq, dk, dk, hd, 100, msl, nh, nkv, 64, ctypes.c_float(1e6), hd, dout, None)
         assert rc == -1
         assert b"1 MiB" in H.lib().yhip_last_error(None)
+
+
+@pytest.mark.parametrize("hd,nh,nkv", [(32, 4, 4), (64, 16, 2), (128, 8, 2)])
+@pytest.mark.parametrize("pos,nsplit", [(0, 0), (319, 0), (320, 0), (2047, 0), (2047, 32), (2112, 33), (4095, 64)])
+def test_noalloc_attention_slice_counts(hd, nh, nkv, pos, nsplit):
+    # One slice (written by the attention itself), two, and 32, 33 and 64 (around the merge launch's first
+    # round of 32 slices and its last): bit for bit the allocating entry point's in-launch merge.
+    H = hip()
+    msl = 4096
+    rng = np.random.default_rng(pos + nsplit + hd)
+    kb, vb = f16(rng.standard_normal(nkv * hd * msl)), f16(rng.standard_normal(nkv * hd * msl))
+    q = rng.standard_normal(nh * hd).astype(np.float32)
+    want, _ = H.attention(q, kb, vb, hd, pos, msl, nh, nkv, nsplit=nsplit)
+    got, k_got = _noalloc(q, kb, vb, hd, pos, msl, nh, nkv, nsplit)
+    assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
+    assert np.array_equal(k_got, kb)

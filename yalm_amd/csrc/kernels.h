@@ -811,6 +811,7 @@ struct AttnArgs {
                           // merged by the next launch (merge_o_kernel) instead of the last slice
   const float* inv_freq;  // [head_dim / 2] rotary frequencies (sink re-rotation by one position)
   const StepParams* params;
+  int pos = 0;            // MFMA kernel as its own launch: the position where params is null
 };
 
 constexpr int kMaxGroup = 8;

@@ -2065,12 +2065,6 @@ extern "C" int yhip_attention_noalloc(const float* q, uint16_t* kcache, const ui
   unsigned char* base = noalloc_scratch();
   if (!base) return YHIP_EDEVICE;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  NaSetup su;
-  su.pos = pos;
-  su.n_freq = head_dim / 2;
-  fill_inv_freq(su.inv_freq, head_dim, rotary_dim, rope_theta);
-  hipLaunchKernelGGL(noalloc_setup_kernel, dim3(1), dim3(64), 0, s, base, su);
-  HIP_TRY(nullptr, hipGetLastError());
   AttnArgs t;
   t.q = q;
   t.kcache = kcache;
@@ -2086,6 +2080,27 @@ extern "C" int yhip_attention_noalloc(const float* q, uint16_t* kcache, const ui
   t.min_slice = min_slice;
   t.inv_freq = reinterpret_cast<const float*>(base + 512);
   t.params = reinterpret_cast<const StepParams*>(base + 256);
+  if (g_attn_mfma && head_dim % 32 == 0 && max_seq_len % 32 == 0 && pos < max_seq_len) {
+    // Matrix-core kernel, no sink rotation: the position goes with the launch, so nothing has to be set
+    // up, and more than one slice is merged by a second launch. Other calls keep the tickets.
+    const int chunk = attn_mfma_chunk(pos + 1, nsplit, min_slice), active = (pos + chunk) / chunk;
+    t.params = nullptr;
+    t.pos = pos;
+    t.defer_merge = active > 1;
+    if (int rc = launch_attention(nullptr, t, s)) return rc;
+    if (active > 1) {
+      hipLaunchKernelGGL(attn_merge_kernel, dim3(n_heads), dim3(kMergeThreads), 0, s, (const float*)t.partial, nsplit,
+                         active, head_dim, att_out);
+      HIP_TRY(nullptr, hipGetLastError());
+    }
+    return YHIP_OK;
+  }
+  NaSetup su;
+  su.pos = pos;
+  su.n_freq = head_dim / 2;
+  fill_inv_freq(su.inv_freq, head_dim, rotary_dim, rope_theta);
+  hipLaunchKernelGGL(noalloc_setup_kernel, dim3(1), dim3(64), 0, s, base, su);
+  HIP_TRY(nullptr, hipGetLastError());
   return launch_attention(nullptr, t, s);
 }
 
