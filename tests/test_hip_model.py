@@ -864,3 +864,22 @@ def test_staged_upload_is_bit_identical():
     with pytest.raises(H.HipError):
         H.set_upload(64, 0)
     H.set_upload()
+
+
+@pytest.mark.parametrize("dim,hd,g,nkv", [(992, 64, 4, 2), (160, 32, 2, 8), (544, 128, 8, 1)])
+def test_attention_and_o_rows_off_their_blocks(dim, hd, g, nkv):
+    # Small models give the O rows four loads per wave instead of sixteen: row blocks of 64, 256 and
+    # 16 rows (8 waves), a half-filled last one, a lone short one and whole ones, on both launches that hold them (attention + O up
+    # to 512 keys, slice merge + O beyond) against the oracle from the same N(0, 1) cache.
+    cfg = dict(MICRO, dim=dim, hidden_dim=256, head_dim=hd, n_heads=g * nkv, n_kv_heads=nkv, rotary_dim=hd,
+               max_seq_len=640)
+    t = np_tensors(cfg, seed=91, std=0.05)
+    om, hm = _models(cfg, t, "graph")
+    prefill = _prefill_kv(om, hm, cfg, np.random.default_rng(92))
+    positions = [5, 300, 511, 512, 600]
+    for pos in positions:
+        lo, lh = om.forward(3, pos), hm.forward(3, pos)
+        # fp16 cache entries that round the other way, as in the one-launch test above
+        assert npref.rel_l2(lh, lo) < 1e-3, pos
+    _check_kv_prefilled(om, hm, cfg, prefill, positions)
+    hm.close()

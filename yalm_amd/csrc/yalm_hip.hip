@@ -380,7 +380,7 @@ int check_attn_shape(yhip_ctx* ctx, int hd, int nh, int nkv) {
 }
 
 // ---- attention + O projection in one launch ------------------------------------------------------
-// Waves per attn_o_kernel workgroup, and its Wo loads per wave: 16 row segments of G*HD columns
+// Waves per attn_o_kernel / merge_o_kernel workgroup, and their Wo loads per wave: 16 row segments of G*HD columns
 // (whole rows of 16-byte chunks), or CPR when a segment has fewer than 64 chunks, so that a wave's
 // rows fit its 64 lanes.
 constexpr int kAttnOWaves = 8;
@@ -388,16 +388,36 @@ template <int HD, int G>
 constexpr int attn_o_loads() {
   return G * HD / 8 >= 16 ? 16 : G * HD / 8;
 }
-template <int HD, int G>
+// Where that leaves half the CUs or more without a workgroup (dim below 4096 with 8 kv heads of 128 x 4: the
+// 1B-class shape, 2048 with heads of 64, has 64 workgroups), a wave takes kAttnOSmall loads instead: four
+// times the workgroups with a quarter of the rows each, the same sums per row. us per decode step there
+// (16 layers) at 50 / 500 / 700 / 3500 keys with 16 loads per wave 541 / 596 / 615 / 654, 8: 518 / 571 / 595 /
+// 628, 4: 510 / 554 / 578 / 609, 2: 522 / 604 / 582 / 617; tiny (dim 256, 4 layers) at 40 keys 92.3, 91.4,
+// 88.4, 87.9.
+constexpr int kAttnOSmall = 4;
+template <int HD, int G, int U>
 int attn_o_blocks(const yhip_config& c) {
-  constexpr int RB = AttnOGeom<HD, G, kAttnOWaves, attn_o_loads<HD, G>()>::RB;
+  constexpr int RB = AttnOGeom<HD, G, kAttnOWaves, U>::RB;
   return c.n_kv_heads * ((c.dim + RB - 1) / RB);
 }
 
+// merge: false = attn_o_kernel (attention inside), true = merge_o_kernel (partials from the attention launch)
 template <int HD, int G>
-void go_attn_o(const yhip_config& c, const AttnArgs& t, const AttnOArgs& o, hipStream_t s) {
-  hipLaunchKernelGGL((attn_o_kernel<HD, G, kAttnOWaves, attn_o_loads<HD, G>()>), dim3(attn_o_blocks<HD, G>(c)),
-                     dim3(64 * kAttnOWaves), 0, s, t, o);
+void go_attn_o(const yhip_config& c, const AttnArgs& t, const AttnOArgs& o, bool merge, int cus, hipStream_t s) {
+  constexpr int U = attn_o_loads<HD, G>();
+  auto go = [&](auto kernel, int blocks) {
+    hipLaunchKernelGGL(kernel, dim3(blocks), dim3(64 * kAttnOWaves), 0, s, t, o);
+  };
+  if constexpr (U > kAttnOSmall) {
+    if (2 * attn_o_blocks<HD, G, U>(c) <= cus) {
+      const int blocks = attn_o_blocks<HD, G, kAttnOSmall>(c);
+      if (merge) go(merge_o_kernel<HD, G, kAttnOWaves, kAttnOSmall>, blocks);
+      else go(attn_o_kernel<HD, G, kAttnOWaves, kAttnOSmall>, blocks);
+      return;
+    }
+  }
+  if (merge) go(merge_o_kernel<HD, G, kAttnOWaves, U>, attn_o_blocks<HD, G, U>(c));
+  else go(attn_o_kernel<HD, G, kAttnOWaves, U>, attn_o_blocks<HD, G, U>(c));
 }
 
 bool attn_o_shape(const yhip_config& c) {
@@ -413,12 +433,6 @@ bool attn_o_at(const yhip_ctx* ctx, int pos) {
          pos + 1 <= ctx->attn_o_max;
 }
 
-template <int HD, int G>
-void go_merge_o(const yhip_config& c, const AttnArgs& t, const AttnOArgs& o, hipStream_t s) {
-  hipLaunchKernelGGL((merge_o_kernel<HD, G, kAttnOWaves, attn_o_loads<HD, G>()>), dim3(attn_o_blocks<HD, G>(c)),
-                     dim3(64 * kAttnOWaves), 0, s, t, o);
-}
-
 // The step at pos leaves the split-KV attention's slice merge to merge_o_kernel when the option is on,
 // the MFMA attention applies and the slices fit the merge kernel's partial block.
 bool split_o_at(const yhip_ctx* ctx, int pos) {
@@ -430,7 +444,7 @@ bool split_o_at(const yhip_ctx* ctx, int pos) {
 // launch)
 int launch_attn_o(yhip_ctx* ctx, const AttnArgs& t, const AttnOArgs& o, hipStream_t s, bool merge = false) {
   const yhip_config& c = ctx->c;
-#define YK_AO(HD, G) (merge ? go_merge_o<HD, G>(c, t, o, s) : go_attn_o<HD, G>(c, t, o, s))
+#define YK_AO(HD, G) go_attn_o<HD, G>(c, t, o, merge, ctx->num_cus, s)
   switch (t.head_dim * 16 + t.n_heads / t.n_kv_heads) {
     case 32 * 16 + 1: YK_AO(32, 1); break;
     case 32 * 16 + 2: YK_AO(32, 2); break;
