@@ -67,12 +67,13 @@ def test_gemm_swiglu(M, N, K, gemm_variant):
 
 
 @pytest.mark.parametrize("M", [1, 31, 33, 64, 65, 96, 97, 128])
-@pytest.mark.parametrize("N,K", [(8, 128), (101, 384), (264, 1664), (16600, 256)])
+@pytest.mark.parametrize("N,K", [(8, 128), (101, 384), (264, 1664), (16600, 256), (11008, 256), (3060, 2048)])
 def test_gemm_weight_streaming(M, N, K):
     # Up to 128 rows with K % 128 == 0: row counts around the kernel's 32-row steps, N around its
     # 16-row tiles and 128-row workgroups (101: rows of outputs that are no multiple of 4), spans of
     # fewer stages than its ring (K 128, 256, 384), 13 stages over 13 splits (264 x 1664: one each;
-    # fp32 partials) and no split (16600 rows: more weight blocks than CUs). fp32 sums of up to 1664
+    # fp32 partials), no split (16600 rows: more weight blocks than CUs) and, on 256 CUs, workgroups of
+    # fewer than eight tiles (SwiGLU 11008: six, 3060 x 2048 without: six, a ragged last one). fp32 sums of up to 2048
     # products: 1e-6 is 16 roundings of the result.
     H = hip()
     assert H.gemm_variant(M, N, K, 0) == (1, 128, (M + 31) // 32 * 32)

@@ -95,6 +95,7 @@ struct GemmArgs {
   float* P;
   long p_floats;  // capacity of P
   int ksplit;     // 0 or 1: no split
+  int tiles;      // weight-streaming kernel: 16-row weight tiles per workgroup, 1..8
   // Split last round of the eight-wave kernel: one flag per partial slot (kSkFlagStride words
   // apart, zeroed once) and the word a timed-out wait sets.
   unsigned* sk_flags;
@@ -358,7 +359,9 @@ __global__ void __launch_bounds__(256) gemm_splitk_reduce(GemmArgs g) {
 // through LDS. v_mfma_f32_16x16x32_f16 with the weights as the A operand: the accumulator holds four
 // consecutive outputs of one activation row (16-byte stores).
 // A wave owns a tile of 16 weight rows (SwiGLU: 8 rows of W1 and the same 8 of W3) times all BM
-// activation rows, a workgroup of eight waves 128 weight rows. A load instruction covers whole 128-byte
+// activation rows, a workgroup of eight waves g.tiles (1..8) of them: the host picks the number that
+// spreads the weights evenly over the CUs (stream_plan), the waves beyond it only copy activations.
+// A load instruction covers whole 128-byte
 // lines, 8 of them per row pair half: lane l reads chunk 2 (l / 16) + (l / 8) % 2 of row l % 8, and
 // the loads of a tile's rows 0-7 and 8-15 are exchanged between lanes l and l ^ 8 (one DPP move per
 // register) into the MFMA's operand, row l % 16 with one k chunk per 16 lanes. In the operand's own
@@ -405,8 +408,8 @@ __device__ __forceinline__ u32x4 swap8(u32x4 keep, u32x4 src) {
   return r;
 }
 
-// Output columns per workgroup.
-constexpr int stream_cols(int epi) { return kStreamWaves * (epi == kGemmSwiGLU ? 8 : 16); }
+// Output columns per wave tile.
+constexpr int stream_cols(int epi) { return epi == kGemmSwiGLU ? 8 : 16; }
 
 template <int EPI, int BM>
 __global__ void __launch_bounds__(64 * kStreamWaves) gemm_stream_kernel(GemmArgs g) {
@@ -416,8 +419,8 @@ __global__ void __launch_bounds__(64 * kStreamWaves) gemm_stream_kernel(GemmArgs
   constexpr int MT = BM / 16;        // 16-row activation tiles
   constexpr int NA = BM / (4 * NW);  // activation copies per wave and stage (4 rows of 256 bytes each)
   constexpr int LPS = NA + 4;        // loads per wave and stage
-  constexpr int TC = EPI == kGemmSwiGLU ? 8 : 16;  // output columns per tile
-  constexpr int NC = stream_cols(EPI);
+  constexpr int TC = stream_cols(EPI);
+  const int NC = g.tiles * TC;       // output columns per workgroup
   __shared__ __attribute__((aligned(1024))) uint16_t As[S][BM * kStreamK];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int ks = g.ksplit > 1 ? g.ksplit : 1;
@@ -433,6 +436,7 @@ __global__ void __launch_bounds__(64 * kStreamWaves) gemm_stream_kernel(GemmArgs
     const int r = 4 * (wave + NW * j) + (lane >> 4);
     arow[j] = g.A + (long)min(r, g.M - 1) * g.lda + 8 * ((lane & 15) ^ (r & 15));
   }
+  const bool live = wave < g.tiles;
   // the wave's weight tile: first output column, and this lane's byte offsets of its two row halves
   const int nb = tn * NC + wave * TC;
   unsigned voff[2];
@@ -447,7 +451,7 @@ __global__ void __launch_bounds__(64 * kStreamWaves) gemm_stream_kernel(GemmArgs
     const int ka = min(st, s1 - 1) * kStreamK;
 #pragma unroll
     for (int j = 0; j < NA; ++j) load_lds16(arow[j] + ka, &As[slot][(wave + NW * j) * 512]);
-    const int kw = st * kStreamK * 2, n = st < s1 ? (int)bytes : 0;
+    const int kw = st * kStreamK * 2, n = live && st < s1 ? (int)bytes : 0;
     const __amdgpu_buffer_rsrc_t r0 =
         __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(g.B), 0, n, kBufferConfig);
     const __amdgpu_buffer_rsrc_t r1 = __builtin_amdgcn_make_buffer_rsrc(
@@ -473,7 +477,7 @@ __global__ void __launch_bounds__(64 * kStreamWaves) gemm_stream_kernel(GemmArgs
     __builtin_amdgcn_sched_barrier(0);
     issue((slot + 3) % S, st + 3);
     __builtin_amdgcn_sched_barrier(0);
-    if (st >= s1) return;
+    if (st >= s1 || !live) return;
 #pragma unroll
     for (int kk = 0; kk < 4; ++kk) {  // line kk / 2, even or odd chunks
       u32x4 fa[MT];
@@ -496,6 +500,7 @@ __global__ void __launch_bounds__(64 * kStreamWaves) gemm_stream_kernel(GemmArgs
     step(3, st + 3);
   }
   wait_vmcnt<0>();  // the copies past the end have landed before the LDS is given back
+  if (!live) return;
 
   // lane l: tile rows 4 (l / 16) .. + 3 of activation row 16 i + l % 16
 #pragma unroll

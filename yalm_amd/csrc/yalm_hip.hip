@@ -954,6 +954,35 @@ void splitk_end(const GemmArgs& g, int* deferred, hipStream_t s) {
                      g);
 }
 
+// Workgroups of the weight-streaming GEMM: 16-row tiles per workgroup and K splits, at most one workgroup
+// per CU (a second one only adds partial sums: W2 at 32 rows 21.6 us with 8 splits, 24.0 with 16). Eight
+// tiles, the widest workgroup, copy the activations the fewest times; fewer (down to four) where that
+// shortens the longest workgroup's rows times k-stages by a quarter, or saves the split at the same
+// length: hidden 11008 172 workgroups of 8 tiles -> 230 of 6, its QKV 96 x 2 splits -> 128 x 2 (us
+// per prefill of 32 / 61 / 128 tokens, 8 layers: 1000 / 1142 / 1434 -> 975 / 1097 / 1376), W1/W3 8192 x
+// 2048 128 x 2 -> 256 of 4 (1B-class 581 / 708 / 920 -> 566 / 685 / 875). For less it does not pay: at the
+// 7B shape W1/W3 in 224 workgroups of 8 tiles 47.6, 256 of 7 48.3 us, QKV in 48 x 5 or 64 x 4 of 6 equal.
+// Returns the workgroups per split.
+long stream_plan(long tiles, int T, long cus, long most_splits, GemmArgs& g) {
+  long best = -1, groups = 0;
+  g.tiles = kStreamWaves;
+  g.ksplit = 1;
+  for (int per = kStreamWaves; per >= kStreamWaves / 2; --per) {
+    const long wgs = (tiles + per - 1) / per;
+    const long ks = std::max(1L, std::min({cus / wgs, (long)T, most_splits}));
+    if (wgs > cus && per < kStreamWaves) break;
+    const long rounds = (wgs * ks + cus - 1) / cus;
+    const long cost = rounds * per * ((T + ks - 1) / ks);
+    if (best < 0 || 4 * cost <= 3 * best || (cost == best && ks == 1 && g.ksplit > 1)) {
+      best = cost;
+      groups = wgs;
+      g.tiles = per;
+      g.ksplit = (int)ks;
+    }
+  }
+  return groups;
+}
+
 // Prefill GEMM launch. The variant is chosen per shape (gemm_choice) unless forced with the
 // process-wide options.
 template <int EPI>
@@ -973,16 +1002,11 @@ int launch_gemm(yhip_ctx* ctx, const GemmArgs& g, hipStream_t s, int* deferred =
     if (e != hipSuccess) return fail(ctx, YHIP_EDEVICE, std::string("gemm launch: ") + hipGetErrorString(e));
     return YHIP_OK;
   }
-  // Weight streaming: one workgroup per CU over (128-row weight blocks x K splits), as many splits as
-  // fit (a second workgroup per CU only adds partial sums: W2 at 32 rows 21.6 us with 8 splits, 24.0
-  // with 16; QKV 12.0 with 5, 14.8 with 10).
   if (stages == 1) {
     GemmArgs ga = g;
-    const long cus = ctx ? ctx->num_cus : device_cus();
-    const long tiles = (g.N + stream_cols(EPI) - 1) / stream_cols(EPI);
     const long part_floats = (long)g.M * g.N * (EPI == kGemmSwiGLU ? 2 : 1);  // per split
-    const long ks = g.P ? std::min({cus / tiles, (long)(g.K / kStreamK), g.p_floats / part_floats}) : 1;
-    ga.ksplit = (int)std::max(1L, ks);
+    const long tiles = stream_plan((g.N + stream_cols(EPI) - 1) / stream_cols(EPI), g.K / kStreamK,
+                                   ctx ? ctx->num_cus : device_cus(), g.P ? g.p_floats / part_floats : 1, ga);
     const dim3 grid(8 * (unsigned)((tiles * ga.ksplit + 7) / 8)), block(64 * kStreamWaves);
     switch (bm) {
       case 32: hipLaunchKernelGGL((gemm_stream_kernel<EPI, 32>), grid, block, 0, s, ga); break;
