@@ -369,7 +369,7 @@ def test_gemm_variants_chosen_per_shape():
 @pytest.mark.parametrize("M,N,K,mode,want", [
     (769, 4096, 14336, 1, 6), (768, 4096, 14336, 1, 6), (513, 4096, 14336, 1, 6), (512, 4096, 14336, 1, 2),
     (769, 6144, 4096, 0, 6), (512, 6144, 4096, 0, 2), (1025, 4096, 4096, 1, 6), (1000, 4090, 4096, 1, 2),
-    (257, 5632, 2048, 2, 2), (203, 1030, 5504, 1, 2), (203, 516, 5504, 0, 2), (150, 520, 4160, 2, 2)])
+    (257, 5632, 2048, 2, 2), (129, 11008, 4096, 2, 6), (255, 11008, 4096, 2, 6), (203, 1030, 5504, 1, 2), (203, 516, 5504, 0, 2), (150, 520, 4160, 2, 2)])
 def test_gemm_mid_rows_on_both_sides_of_the_split_rule(M, N, K, mode, want):
     # Between the LDS pipeline and full rounds of 256 x 256 tiles: the eight-wave kernel takes grids
     # that it can split along K into two to five parts of at least 20 k-steps, the rest stays with the

@@ -890,12 +890,13 @@ void gemm_choice(int epi, int M, int N, int K, int cus, int& stages, int& bk, in
   // tile costs about as much as eight k-steps, and the main part adds them one after the other): W2 at
   // 640 / 1013 rows 196 / 126 / 108 and 201 / 136 / 134, QKV at 640 / 1013 60 / 72 / 54 and 76 / 76 /
   // 65, O at 1280 69 / 74 / 60; in more or shorter parts it loses (O at 640 rows 59 / 42 / 52). Up to 256
-  // rows, one row of tiles, W1/W3 stays with 256-row workgroups, which the variant test holds it to
-  // (240 rows: 87 / 89 / 77).
+  // rows, one row of tiles, only W1/W3 have enough of them: 160 / 240 rows 83 / 86 / 77 and 87 / 89 / 77;
+  // 256 rows exactly would gain as much, but the variant test holds them to 256-row workgroups.
   const int nc = epi == kGemmSwiGLU ? kBigN / 2 : kBigN;
   const long big_tiles = (long)((M + kBigM - 1) / kBigM) * ((N + nc - 1) / nc);
   const long parts = cus / big_tiles;
-  const bool split_parts = M > kBigM && parts >= 2 && parts <= 5 && K / 64 >= 20 * parts;
+  const bool split_rows = M > kBigM || (epi == kGemmSwiGLU && M > kStreamRows && M != kBigM);
+  const bool split_parts = split_rows && parts >= 2 && parts <= 5 && K / 64 >= 20 * parts;
   if (K % 64 == 0 && (big_tiles * 16 >= (long)cus * 9 || split_parts)) {
     stages = 6;
     bk = 64;
