@@ -241,15 +241,17 @@ def test_prefill_in_chunks_and_after_decode_steps():
 
 
 @pytest.mark.parametrize("start,n", [(223, 5), (224, 5), (255, 33), (701, 1), (960, 64), (901, 90)])
-@pytest.mark.parametrize("shape", ["hd32_g1", "hd64_g2", "hd128_g4", "hd32_g8"])
+@pytest.mark.parametrize("shape", ["hd32_g1", "hd64_g2", "hd128_g4", "hd32_g8", "hd32_3heads"])
 def test_prefill_key_split_behind_a_long_context(shape, start, n):
     # Few queries behind a long cache: the keys are split over workgroups from two parts of four
     # 32-key tiles on (224 cached positions), each part's sums merged by their maxima. Starts on and
     # off the tile and split edges, one query, a full and a ragged query block, every count of query
-    # heads per kv head, against the oracle's steps from the same N(0, 1) cache. Weights of std 0.1
-    # make the attention a large part of every layer's output.
-    hd, g = {"hd32_g1": (32, 1), "hd64_g2": (64, 2), "hd128_g4": (128, 4), "hd32_g8": (32, 8)}[shape]
-    cfg = dict(MICRO, dim=256, hidden_dim=256, head_dim=hd, n_heads=2 * g, n_kv_heads=2, rotary_dim=hd,
+    # heads per kv head, against the oracle's steps from the same N(0, 1) cache. An odd number of heads
+    # leaves the (max, sum) pairs at sizes that are no multiple of the parts' 16-byte stores. Weights
+    # of std 0.1 make the attention a large part of every layer's output.
+    hd, g, nkv = {"hd32_g1": (32, 1, 2), "hd64_g2": (64, 2, 2), "hd128_g4": (128, 4, 2), "hd32_g8": (32, 8, 2),
+                  "hd32_3heads": (32, 1, 3)}[shape]
+    cfg = dict(MICRO, dim=256, hidden_dim=256, head_dim=hd, n_heads=nkv * g, n_kv_heads=nkv, rotary_dim=hd,
                max_seq_len=1024)
     t = np_tensors(cfg, seed=71, std=0.1)
     om = O.OracleModel(cfg, t)

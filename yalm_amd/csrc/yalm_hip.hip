@@ -1067,7 +1067,7 @@ int launch_gemm(yhip_ctx* ctx, const GemmArgs& g, hipStream_t s, int* deferred =
 constexpr int kSplitTiles = 4;
 int prefill_attn_splits(const PrefillAttnArgs& p, int head_dim, int units, int cus, long p_floats) {
   const long per = (long)p.n * p.n_heads * (head_dim + 2);  // floats per split
-  const long most = std::min({(long)(cus / units), (long)(p.start / 32 + 1) / kSplitTiles, p_floats / per});
+  const long most = std::min({(long)(cus / units), (long)(p.start / 32 + 1) / kSplitTiles, (p_floats - 4) / per});
   return (int)std::max(1L, most);
 }
 
@@ -1084,7 +1084,7 @@ bool launch_prefill_attn_hd(PrefillAttnArgs p, int G, int n_qtiles, float* ws, l
       return;
     }
     p.part_ml = (float2*)ws;
-    p.part_o = ws + 2L * p.splits * p.n * p.n_heads;
+    p.part_o = ws + (2L * p.splits * p.n * p.n_heads + 3) / 4 * 4;  // 16-byte aligned
     hipLaunchKernelGGL(split_kernel, dim3(units * p.splits), dim3(threads), 0, s, p);
     hipLaunchKernelGGL(prefill_attn_merge_kernel, dim3(p.n, (p.n_heads * HD + 4 * kBlock - 1) / (4 * kBlock)),
                        dim3(kBlock), 0, s, p, HD);
