@@ -85,11 +85,13 @@ def micro_bytes(kind, rows, cols, norm, resid):
 
 def prefill_flops(cfg, n, start=0):
     """Dense matmul FLOPs of n prompt tokens through every layer (2 per weight per token) plus the
-    causal attention (QK^T and PV: 4 * head_dim * n_heads per key-query pair)."""
+    causal attention (QK^T and PV: 4 * head_dim * n_heads per key-query pair), as the prefill runs
+    them: behind the last layer's QKV only the last token goes on (the lm_head reads nothing else)."""
     d, hid, hd, nh, nkv = cfg["dim"], cfg["hidden_dim"], cfg["head_dim"], cfg["n_heads"], cfg["n_kv_heads"]
-    w_layer = (nh * hd + 2 * nkv * hd) * d + d * nh * hd + 3 * d * hid
+    w_qkv, w_rest = (nh * hd + 2 * nkv * hd) * d, d * nh * hd + 3 * d * hid
     pairs = sum(start + i + 1 for i in range(n))
-    return cfg["n_layers"] * (2.0 * n * w_layer + 4.0 * hd * nh * pairs)
+    L = cfg["n_layers"]
+    return 2.0 * L * n * w_qkv + 2.0 * ((L - 1) * n + 1) * w_rest + 4.0 * hd * nh * ((L - 1) * pairs + start + n)
 
 
 def log(*a):
