@@ -123,6 +123,24 @@ def test_matvec_row_lengths_at_the_piece_edges(n, d):
     assert np.array_equal(hip().matvec(x, w), np.where(np.arange(d) % 2, np.inf, -np.inf))
 
 
+@pytest.mark.parametrize("n", [8, 256, 504, 520, 1032, 2056, 4104, 11008])
+@pytest.mark.parametrize("d", [5, 6, 1030])
+@pytest.mark.parametrize("nan", [0, 1])
+def test_matvec_rows_end_where_the_next_row_begins(n, d, nan):
+    # Row lengths that do not fill the streamed pieces, single rows (odd d) and pairs, with every other
+    # row all NaN (the first or the second one): a load past a row's end would meet a zero input, and
+    # 0 * NaN is NaN. The other rows are bit for bit what they are beside finite rows.
+    rng = np.random.default_rng(n + d)
+    w = f16(rng.standard_normal((d, n)) * 0.05)
+    x = rng.standard_normal(n).astype(np.float32)
+    want = hip().matvec(x, w)
+    assert np.isfinite(want).all()
+    w[nan::2] = 0x7E00  # fp16 NaN
+    got = hip().matvec(x, w)
+    assert np.isnan(got[nan::2]).all()
+    assert np.array_equal(got[1 - nan::2], want[1 - nan::2])
+
+
 @pytest.mark.parametrize("dim,hidden", [(64, 128), (256, 768), (4096, 14336)])
 @pytest.mark.parametrize("act", [1, 0])
 def test_ffn_parity(dim, hidden, act, bpc):

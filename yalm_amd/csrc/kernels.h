@@ -592,7 +592,8 @@ __global__ void __launch_bounds__(kBlock) matvec_kernel(MatvecArgs a) {
 // ------------------------------------------------------------------------------------------
 // The same matvec for any row length K <= 1024*NPT (K % 8 == 0): rows are streamed in pieces of KC
 // chunks per lane, the last piece cut by the buffer descriptor's size (a load past the row returns
-// zero without a memory access), so the pipeline of matvec_body (two register buffers, the next
+// zero without a memory access: the range check covers the vector and instruction offsets only, so a
+// chunk's offset goes there and the scalar one stays 0), so the pipeline of matvec_body (two register buffers, the next
 // piece issued before the current one is used, staging reads ahead of the first weights) holds for
 // every model width and not only for the unrolled 4096 and 14336. MULTI: rows of more than one piece.
 // A lane's chunk past the row multiplies its zero weights by the zero chunk at lds + 8, never by
@@ -662,7 +663,7 @@ __device__ __forceinline__ RowMax matvec_any_body(const MatvecArgs& a, int blk, 
           const_cast<uint16_t*>(rows[r]) + done / 2, 0, left, kBufferConfig);
 #pragma unroll
       for (int u = 0; u < KC; ++u)
-        wv[r][u] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, lane * 16, u * 1024, kCpolNt));
+        wv[r][u] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, lane * 16 + u * 1024, 0, kCpolNt));
     }
     epilogue_prefetch<R, EPI>(a, g, pre);
     if (!MULTI || ++ip == np) {
