@@ -91,6 +91,25 @@ def test_gemm_weight_streaming(M, N, K):
     assert npref.rel_l2(got, want / (1 + np.exp(-want)) * u) < 2e-3  # fp16 output
 
 
+@pytest.mark.parametrize("M", [1, 40, 100])
+@pytest.mark.parametrize("N,K", [(24, 128), (101, 384), (264, 1664), (40, 4096)])
+def test_gemm_weight_streaming_columns_do_not_mix(M, N, K):
+    # Every other weight row all NaN (and, for SwiGLU, the same rows of both weights): the outputs of the
+    # others are bit for bit what they are beside finite rows, with spans shorter than the ring of stages
+    # (K 128, 384 and the K splits of 264 x 1664), whose stages past the end load no weights.
+    H = hip()
+    rng = np.random.default_rng(M + N + K)
+    a = f16(rng.standard_normal((M, K)))
+    b = f16(rng.standard_normal((N, K)) * 0.05)
+    b3 = f16(rng.standard_normal((N, K)) * 0.05)
+    want = [H.gemm(a, b, mode=0), H.gemm(a, b, mode=2, b3=b3)]
+    b[1::2] = b3[1::2] = 0x7E00  # fp16 NaN
+    for w, got in zip(want, [H.gemm(a, b, mode=0), H.gemm(a, b, mode=2, b3=b3)]):
+        assert np.array_equal(got[:, ::2], w[:, ::2])
+        bad = got[:, 1::2] if got.dtype == np.float32 else h2f(got[:, 1::2])
+        assert np.isnan(bad).all()
+
+
 @pytest.mark.parametrize("ksplit", [2, 4, 8])
 @pytest.mark.parametrize("M,N,K", [(37, 192, 1024), (128, 256, 4096), (200, 128, 512)])
 def test_gemm_split_k(M, N, K, ksplit):

@@ -371,8 +371,9 @@ __global__ void __launch_bounds__(256) gemm_splitk_reduce(GemmArgs g) {
 // Each stage orders its activation copies (global_load_lds, [BM][128] halves with chunk c of row r
 // at position c ^ (r % 16): the 16 rows of a fragment read fall in distinct banks) before its weight
 // loads, so one vmcnt wait covers both and the barrier behind it publishes the activations. Stages
-// past the end re-read the last activations and load weights through an empty descriptor, so every
-// iteration has the same loads in flight.
+// past the end re-read the last activations and load weights through an empty descriptor (at the last
+// stage's offsets: the scalar offset takes no part in the range check, so it stays inside the weights by
+// itself), so every iteration has the same loads in flight.
 // K % 128 == 0. Against the LDS pipeline (which keeps one 16 KB weight stage per workgroup in flight),
 // us per launch in a 7B prefill: 32 rows W1/W3 68.0 -> 45.7 (5.1 TB/s), W2 32.1 -> 22.1, QKV 19.2 -> 12.6,
 // O 15.2 -> 10; 61 rows 69.2 -> 48.7, 34.0 -> 25.9, 20.6 -> 15.8. What is left above the pattern's
@@ -448,10 +449,10 @@ __global__ void __launch_bounds__(64 * kStreamWaves) gemm_stream_kernel(GemmArgs
   const unsigned bytes = (unsigned)g.N * (unsigned)(g.ldb * 2);
   u32x4 w[S][2][2];  // [slot][128-byte line][row half]
   auto issue = [&](int slot, int st) {
-    const int ka = min(st, s1 - 1) * kStreamK;
+    const int ka = min(st, s1 - 1) * kStreamK;  // past the end: the last stage's addresses again
 #pragma unroll
     for (int j = 0; j < NA; ++j) load_lds16(arow[j] + ka, &As[slot][(wave + NW * j) * 512]);
-    const int kw = st * kStreamK * 2, n = live && st < s1 ? (int)bytes : 0;
+    const int kw = ka * 2, n = live && st < s1 ? (int)bytes : 0;
     const __amdgpu_buffer_rsrc_t r0 =
         __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(g.B), 0, n, kBufferConfig);
     const __amdgpu_buffer_rsrc_t r1 = __builtin_amdgcn_make_buffer_rsrc(
