@@ -600,10 +600,13 @@ __global__ void __launch_bounds__(kBlock) matvec_kernel(MatvecArgs a) {
 // whatever follows the input in LDS.
 // What it replaces (a rolled loop that waited for every 1 KB load before the next one, the input
 // staged before the first weights) was bound by that wait. Measured on MI355X, weights rotating
-// through 1 GiB, µs per launch before -> after (and TB/s): W2 4096 x 11008 48.2 -> 16.0 (5.6), W2
-// 2048 x 8192 18.8 -> 7.4 (4.5), W2 5120 x 13824 71.0 -> 23.8 (6.0), W1/W3 8192 x 2048 13.7 -> 12.2
-// (5.5), QKV 7168 x 5120 19.7 -> 14.6 (5.0), lm_head 32000 x 2048 27.8 -> 20.7 (6.3).
+// through 1 GiB, µs per launch before -> after (and TB/s): W2 4096 x 11008 48.2 -> 16.1 (5.6), W2
+// 2048 x 8192 19.0 -> 7.2 (4.7), W2 5120 x 13824 71.2 -> 23.6 (6.0), W1/W3 8192 x 2048 13.7 -> 11.8
+// (5.7), QKV 7168 x 5120 19.8 -> 14.9 (4.9), lm_head 32000 x 2048 27.4 -> 20.8 (6.3).
 // ------------------------------------------------------------------------------------------
+// Rows of up to 512 columns have an instantiation of one chunk per lane (KC = 1): with two, the second
+// load and the second dot product of every row were all zeros (O 4096 x 512 of a tensor-parallel shard 3.44 ->
+// 3.35 us a launch, lm_head 32000 x 256 6.4 -> 5.5).
 constexpr int any_chunks(int npt) { return npt >= 4 ? 8 : 2 * npt; }
 
 template <int NPT, bool GAIN, bool EMB>
@@ -633,9 +636,8 @@ __device__ __forceinline__ void stage_load_any(const MatvecArgs& a, StagedInput<
   st.rc = a.rope_cs && (int)threadIdx.x < a.head_dim ? a.rope_cs[threadIdx.x] : 0.f;
 }
 
-template <int R, EpiKind EPI, int NPT>
+template <int R, EpiKind EPI, int NPT, int KC>
 __device__ __forceinline__ RowMax matvec_any_body(const MatvecArgs& a, int blk, int nblk, float* lds) {
-  constexpr int KC = any_chunks(NPT);
   constexpr bool MULTI = NPT > 4;  // K > 512 * KC
   float* red = lds;                // kWavesPerBlock floats; floats 8..15 stay zero
   float* xs = lds + 16;            // K floats (+ the RoPE table)
@@ -644,10 +646,8 @@ __device__ __forceinline__ RowMax matvec_any_body(const MatvecArgs& a, int blk, 
   RowMax mx;
   const uint16_t* x16 = embedding_input(a, blk);
   const int p0 = blk * kWavesPerBlock + __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-  const int n = p0 < a.groups ? (a.groups - 1 - p0) / wave_stride + 1 : 0;  // this wave's groups
   const int nch = a.K >> 3;
   const int np = MULTI ? (nch + kWave * KC - 1) / (kWave * KC) : 1;  // pieces per row
-  const int items = n * np;
   u32x4 wa[R][KC], wb[R][KC];
   float prea[R], preb[R];
   int ig = 0, ip = 0;  // group and piece of the next issue
@@ -674,7 +674,11 @@ __device__ __forceinline__ RowMax matvec_any_body(const MatvecArgs& a, int blk, 
   StagedInput<NPT, kEpiGain<EPI>, kEpiEmb<EPI>> st;
   stage_load_any(a, st, x16);
   __builtin_amdgcn_sched_barrier(0);
-  issue(wa, prea, n > 0);  // unconditional: a branch here would make the staging wait for it
+  issue(wa, prea, p0 < a.groups);  // unconditional: a branch here would make the staging wait for it
+  __builtin_amdgcn_sched_barrier(0);
+  // this wave's pieces, all groups: a division, so behind the first loads, which need only p0 < groups (O
+  // 4096 x 512 3.35 -> 3.06 us, the rolled loop before 3.28)
+  const int items = p0 < a.groups ? ((a.groups - 1 - p0) / wave_stride + 1) * np : 0;
   const int pos = EPI == kEpiQkvRope ? (a.pos >= 0 ? a.pos : a.params->pos) : 0;
   if (threadIdx.x < 8) lds[8 + threadIdx.x] = 0.f;
   stage_store<true>(a, st, xs, red, x16);
@@ -720,10 +724,10 @@ __device__ __forceinline__ RowMax matvec_any_body(const MatvecArgs& a, int blk, 
   return mx;
 }
 
-template <int R, EpiKind EPI, int NPT>
+template <int R, EpiKind EPI, int NPT, int KC = any_chunks(NPT)>
 __global__ void __launch_bounds__(kBlock) matvec_any_kernel(MatvecArgs a) {
   extern __shared__ float lds[];
-  matvec_any_body<R, EPI, NPT>(a, blockIdx.x, gridDim.x, lds);
+  matvec_any_body<R, EPI, NPT, KC>(a, blockIdx.x, gridDim.x, lds);
 }
 
 // Packed (logit, index) whose unsigned order is the argmax order with the reference's tie rule
@@ -762,10 +766,10 @@ __global__ void __launch_bounds__(kBlock) lm_head_argmax_kernel(MatvecArgs a, un
   const RowMax mx = matvec_body<KC, 2, kEpiStore>(a, blockIdx.x, gridDim.x, lds);
   argmax_post(mx, key);
 }
-template <int NPT>
+template <int NPT, int KC = any_chunks(NPT)>
 __global__ void __launch_bounds__(kBlock) lm_head_argmax_any_kernel(MatvecArgs a, unsigned long long* key) {
   extern __shared__ float lds[];
-  const RowMax mx = matvec_any_body<2, kEpiStore, NPT>(a, blockIdx.x, gridDim.x, lds);
+  const RowMax mx = matvec_any_body<2, kEpiStore, NPT, KC>(a, blockIdx.x, gridDim.x, lds);
   argmax_post(mx, key);
 }
 

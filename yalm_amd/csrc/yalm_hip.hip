@@ -217,10 +217,10 @@ std::vector<float> make_inv_freq(int head_dim, int rotary_dim, float theta) {
 // That balances the launch's tail (2.621 -> 2.570 ms per token); 2-8 per CU are in between, 14 and 16
 // no better.
 // Other row lengths (matvec_any_kernel): one workgroup per CU from 2048 columns on, so the input is
-// staged once per CU (µs with 1 / 2 / 12 per CU: QKV 7168 x 5120 14.6 / 15.6 / 16.1, W1/W3 13824 x 5120
-// 44.4 / 44.6 / 48.0, W1/W3 8192 x 2048 12.2 / 12.4 / 12.6, W2 2048 x 8192 7.4 / 7.9 / 7.9), four on
+// staged once per CU (µs with 1 / 2 / 12 per CU: QKV 7168 x 5120 15.0 / 16.1 / 16.6, W1/W3 13824 x 5120
+// 44.7 / 45.2 / 46.3, W1/W3 8192 x 2048 11.9 / 12.1 / 12.3, W2 2048 x 8192 7.3 / 7.8 / 7.8), four on
 // shorter rows, whose staging is nothing beside the waves' own latency (lm_head 32000 x 256 with
-// 1 / 2 / 4 / 12: 9.6 / 7.2 / 6.6 / 7.3).
+// 1 / 2 / 4 / 12: 8.5 / 6.7 / 5.4 / 6.1).
 int default_bpc(int K, int kind = -1) {
   if (K == 4096) return kind == kEpiSwiGLU ? 12 : 2;
   return K >= 2048 ? 1 : 4;
@@ -233,12 +233,14 @@ void launch_mv(const MatvecArgs& a, int blocks, hipStream_t s) {
   hipLaunchKernelGGL((matvec_kernel<KC, R, EPI, H>), dim3(blocks), dim3(kBlock), lds, s, a);
 }
 
-// Row lengths other than the unrolled ones: the smallest staging (NPT float4 per thread) that holds K.
+// Row lengths other than the unrolled ones: the smallest staging (NPT float4 per thread) that holds K, and
+// one chunk per lane where that covers the row.
 template <int R, EpiKind EPI>
 void launch_mv_any(const MatvecArgs& a, int blocks, hipStream_t s) {
   const size_t lds = (16 + (size_t)a.K + (a.rope_cs ? (size_t)a.head_dim : 0)) * sizeof(float);
   auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3(blocks), dim3(kBlock), lds, s, a); };
-  if (a.K <= 1024) go(matvec_any_kernel<R, EPI, 1>);
+  if (a.K <= 512) go(matvec_any_kernel<R, EPI, 1, 1>);
+  else if (a.K <= 1024) go(matvec_any_kernel<R, EPI, 1>);
   else if (a.K <= 2048) go(matvec_any_kernel<R, EPI, 2>);
   else if (a.K <= 4096) go(matvec_any_kernel<R, EPI, 4>);
   else if (a.K <= 8192) go(matvec_any_kernel<R, EPI, 8>);
@@ -608,6 +610,7 @@ int enqueue_step(yhip_ctx* ctx, int mode, int variant) {
       hipLaunchKernelGGL(kernel, dim3(blocks), dim3(kBlock), lds, s, a, ctx->argmax_key);
     };
     if (a.K == 4096) go(lm_head_argmax_kernel<8>);
+    else if (a.K <= 512) go(lm_head_argmax_any_kernel<1, 1>);
     else if (a.K <= 1024) go(lm_head_argmax_any_kernel<1>);
     else if (a.K <= 2048) go(lm_head_argmax_any_kernel<2>);
     else if (a.K <= 4096) go(lm_head_argmax_any_kernel<4>);
