@@ -259,6 +259,23 @@ def test_prefill_in_chunks_and_after_decode_steps():
     hm.close()
 
 
+def test_prefill_rotates_every_pair_alike():
+    # With theta 1 every rotary pair turns by the same angle, so two pairs of a head with the same weight
+    # rows hold the same keys to the last bit, whichever lane and register they pass through (a product of
+    # the rotation rounded in one and fused in the other shows in one fp16 key of some ten thousand).
+    cfg = dict(MICRO, dim=256, hidden_dim=256, n_layers=1, head_dim=128, rotary_dim=128, n_heads=8, n_kv_heads=4,
+               rope_theta=1.0, max_seq_len=2048)
+    t = np_tensors(cfg, seed=101, std=0.1)
+    wk = t["model.layers.0.attn.wk.weight"].reshape(-1, 4, cfg["dim"])  # quads of rows: two pairs each
+    wk[:, 2:] = wk[:, :2]
+    hm = hip().HipModel(cfg, t)
+    toks = np.random.default_rng(102).integers(0, cfg["vocab_size"], 2000)
+    hm.prefill(toks, logits=False)
+    k = np.asarray(hm.kv(0)[0]).reshape(4, 128 // 16, 2048, 4, 4)[:, :, :2000]  # [g][chunk][t][quad][dim]
+    assert np.array_equal(k[..., 2:], k[..., :2])
+    hm.close()
+
+
 @pytest.mark.parametrize("start,n", [(223, 5), (224, 5), (255, 33), (701, 1), (960, 64), (901, 90)])
 @pytest.mark.parametrize("shape", ["hd32_g1", "hd64_g2", "hd128_g4", "hd32_g8", "hd32_3heads"])
 def test_prefill_key_split_behind_a_long_context(shape, start, n):

@@ -1009,8 +1009,10 @@ __device__ __forceinline__ void qk_row(const QkvRowsArgs& a, int t, int part, fl
       for (int e = 0; e < 4; e += 2) {
         const float v0 = clipf(v[e], a.qkv_clip), v1 = clipf(v[e + 1], a.qkv_clip);
         const float cs = rope[j + e], sn = rope[j + e + 1];
-        v[e] = v0 * cs - v1 * sn;
-        v[e + 1] = v0 * sn + v1 * cs;
+        // which product is rounded is written out: left to the compiler, it differed from one pair of a
+        // quad to the other and changed with the code around
+        v[e] = fmaf(v0, cs, -(v1 * sn));
+        v[e + 1] = fmaf(v1, cs, v0 * sn);
       }
     }
     const float amax = group_max(fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3]))), hq);
