@@ -293,8 +293,8 @@ __global__ void __launch_bounds__(BM * 2) gemm_lds_kernel(GemmArgs g) {
       }
   } else {
     // through buffer accesses bounded to the tile, as the eight-wave kernel's epilogue: the residual's
-    // loads go out 32 at a time (guarded read-modify-writes took one memory round trip each: O at 640
-    // rows 65.4 -> 46.4 us, at 1013 70.1 -> 51.2)
+    // loads go out 32 at a time (guarded read-modify-writes took one memory round trip each: O at 1013
+    // rows, in traces of whole prefills, 79.3 -> 64.3 us)
     const int rows = min(BM, g.M - m0);
     constexpr unsigned kOut = 0x80000000u;  // a byte offset past any tile's buffer
     const __amdgpu_buffer_rsrc_t cr =

@@ -273,9 +273,9 @@ int default_attn_splits(int cus, int n_kv_heads) {
   return std::max(1, std::min(64, 7 * cus / (8 * std::max(1, n_kv_heads))));
 }
 
-// Split-K workspace bound: tiles x splits never exceed one workgroup per CU, and a 128 x 128 tile
-// (or 128 x 64 of W1 and of W3) holds 16384 partial sums; the eight-wave GEMM's split last round
-// keeps one 256 x 256 fp32 slot per CU.
+// Capacity of the prefill's partial sums: one 256 x 256 fp32 slot per CU, what the eight-wave GEMM's split
+// last round takes at most. The other users (the K splits of the LDS pipeline and of the streaming GEMM, the
+// key splits of the attention) cut their number of splits to what fits, from p_floats at the launch.
 long splitk_ws_floats(int cus) { return (long)cus * kSkSlotFloats; }
 // Split-last-round flags: one word per CU slot, kSkFlagStride words apart.
 size_t sk_flag_bytes(int cus) { return (size_t)cus * kSkFlagStride * sizeof(unsigned); }
@@ -830,10 +830,9 @@ int run_step_inner(yhip_ctx* ctx, int token, int pos, int mode) {
 // five whole rounds, 80 tail workers of up to 3 pieces, kd 48 of 64 k-steps); with fewer, S parts
 // per tile (S = CUs / tiles, at most 8, pieces of at least 8 k-steps) run side by side (QKV at
 // 3200 rows: 56 tiles, 4 parts each). A grid of fewer tiles than CUs but more than half of them
-// (W2 and O at 3200 rows: 208) is not split: filling the idle CUs slowed every main part by ~10%
-// (the GPU is at its power limit), measured neutral for W2 and 16% slower for O. No split without
-// the partial workspace, when the round is full, or when the pieces would be too small or too
-// many per worker.
+// (W2 and O at 3200 rows: 208) is not split: filling the idle CUs slowed every main part by ~10%,
+// measured neutral for W2 and 16% slower for O. No split without the partial workspace, when the
+// round is full, or when the pieces would be too small or too many per worker.
 PPSplit pp_split_plan(long tiles, int KI, int P, bool workspace) {
   PPSplit sp{};
   sp.dp = 8 * (int)((tiles + 7) / 8);
@@ -893,8 +892,10 @@ void gemm_choice(int epi, int M, int N, int K, int cus, int& stages, int& bk, in
   // tile costs about as much as eight k-steps, and the main part adds them one after the other): W2 at
   // 640 / 1013 rows 196 / 126 / 108 and 201 / 136 / 134, QKV at 640 / 1013 60 / 72 / 54 and 76 / 76 /
   // 65, O at 1280 69 / 74 / 60; in more or shorter parts it loses (O at 640 rows 59 / 42 / 52). Up to 256
-  // rows, one row of tiles, only W1/W3 have enough of them: 160 / 240 rows 83 / 86 / 77 and 87 / 89 / 77;
-  // 256 rows exactly would gain as much, but the variant test holds them to 256-row workgroups.
+  // rows, one row of tiles, only W1/W3 have enough of them: 130 / 200 / 255 rows 81 / 81 / 73, 79 / 81 / 72
+  // and 85 / 81 / 73; whole prefills of 130 / 160 / 200 / 230 rows 0.5 / 0.7 / 2 / 3% shorter (hidden 11008
+  // 1.3 / 1.4 / 2.5 / 4.3%). 256 rows exactly would gain as much (85 / 81 / 72), but the variant test holds
+  // them to 256-row workgroups.
   const int nc = epi == kGemmSwiGLU ? kBigN / 2 : kBigN;
   const long big_tiles = (long)((M + kBigM - 1) / kBigM) * ((N + nc - 1) / nc);
   const long parts = cus / big_tiles;
@@ -912,8 +913,10 @@ void gemm_choice(int epi, int M, int N, int K, int cus, int& stages, int& bk, in
   // own (QKV at 240 / 450 rows 36 / 26 and 60 / 44, O 23 / 20 and 35 / 27, at 768 60 / 43) and their own
   // split leaves at least six k-steps to each part (QKV 3072 x 2048 and O 2048 x 2048 at 240 rows, 3 and 2
   // k-steps: 16.2 / 15.1 and 15.5 / 15.2, but twice the partial sums to add, 128 / 134 us per layer). O
-  // from 897 to 1024 rows, a full round of 128-row tiles, is held to those by the variant test, 62 / 44,
-  // and so is QKV at 200 rows, which puts the line for a short K right above that.
+  // from 897 to 1024 rows, a full round of 128-row tiles, is held to those by the variant test, 61 / 42
+  // (9 us of the difference go back into adding the two splits behind it), and so is QKV at 200 rows, which
+  // puts the line for a short K right above that although 129 to 200 rows would gain too (QKV at 130 / 160 /
+  // 200 rows 35 / 23, 34 / 22 and 34 / 23, O 22 / 18, 21 / 17 and 21 / 18).
   const long tiles = (long)((M + kGBM - 1) / kGBM) * ((N + kGBN - 1) / kGBN);
   const long tiles_big = (long)((M + kBigM - 1) / kBigM) * ((N + kGBN - 1) / kGBN);
   const long steps = K / 64 / std::max(1L, cus / tiles_big);  // k-steps per part with 256-row workgroups
