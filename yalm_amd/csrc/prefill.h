@@ -888,7 +888,7 @@ __global__ void __launch_bounds__(kBlock) rmsnorm_rows_kernel(const float* X, co
 // split order, and, with a gain, the next product's Xn[t] = fp16(rmsnorm(X[t])) in the same pass. One
 // launch and one trip of X instead of two, and 1024 threads to a row, so that all of a row's loads are
 // one round trip deep: 4.8 + 4.7 -> 4.7 us after
-// O and after W2 at 32 rows of the 7B shape, 6.5 + 4.8 -> 6.4 at 203 (256 threads to a row: 7.0 and 9.1).
+// O and after W2 at 32 rows of the 7B shape, 6.5 + 4.8 -> 6.4 at 203 with 4 splits, 7.4 with 8 (256 threads to a row: 7.0 and 9.1).
 // dim % 4 == 0 and dim <= 16384 (prefill_supported, yhip_create).
 constexpr int kRowThreads = 1024;
 __global__ void __launch_bounds__(kRowThreads) splitk_resid_norm_kernel(const float* P, int ksplit, int n, float* X,
@@ -1076,7 +1076,7 @@ __device__ __forceinline__ void v_rows(const QkvRowsArgs& a, int p0, int d0, uin
 // Both parts in one launch: q_blocks workgroups per row, then one per 64 x 64 tile of v. Few rows take
 // several workgroups each (q_blocks), so that the launch is one memory round trip deep and not one per
 // 1024 columns: 32 rows of the 7B shape behind 5 K splits 4.8 + 5.9 + 4.8
-// us (reduce, q and k, v) -> 4.8, 3200 rows (no split) 22.4 + 5.5 -> 24.1.
+// us (reduce, q and k, v) -> 4.8, 3200 rows (no split) 22.4 + 5.5 -> 25.3.
 __global__ void __launch_bounds__(kBlock) qkv_rows_kernel(QkvRowsArgs a) {
   __shared__ union {
     float rope[128];  // (cos, sin) per rotary pair; head_dim <= 128 on the batched path (prefill_supported)
@@ -1132,7 +1132,7 @@ struct PrefillAttnArgs {
 // that key 32 * j0 of every part precedes every query of the block and its running maximum is finite
 // from the first tile on; the last part also takes the tiles from there to the block's last query.
 // 61 queries behind 3001 positions (7B shape: 8 workgroups and a chain of 96 tiles unsplit, 120
-// workgroups of 6 split): 87.4 -> 21.2 + 7.5 us (merge) per layer.
+// workgroups of 6 split): 87.4 -> 19.5 + 8.9 us (merge) per layer.
 template <int HD, int G, int QT, bool SPLIT = false>
 __global__ void __launch_bounds__(64 * G * QT) prefill_attn_kernel(PrefillAttnArgs a) {
   static_assert(HD % 32 == 0, "head_dim must be a multiple of 32");
