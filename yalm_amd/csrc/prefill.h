@@ -1131,8 +1131,8 @@ struct PrefillAttnArgs {
 // A key split starts no later than the tile of the block's first query (start / 32 + 1 >= splits), so
 // that key 32 * j0 of every part precedes every query of the block and its running maximum is finite
 // from the first tile on; the last part also takes the tiles from there to the block's last query.
-// 61 queries behind 3001 positions (7B shape: 8 workgroups and a chain of 96 tiles unsplit, 120
-// workgroups of 6 split): 87.4 -> 19.5 + 8.9 us (merge) per layer.
+// 61 queries behind 3001 positions (7B shape: 8 workgroups and a chain of 96 tiles unsplit, 184
+// workgroups of 4 split): 87.4 -> 19.5 + 8.9 us (merge) per layer.
 template <int HD, int G, int QT, bool SPLIT = false>
 __global__ void __launch_bounds__(64 * G * QT) prefill_attn_kernel(PrefillAttnArgs a) {
   static_assert(HD % 32 == 0, "head_dim must be a multiple of 32");
